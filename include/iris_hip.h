@@ -77,12 +77,13 @@ uint64_t q8gpu_workspace_bytes(const Q8GpuMatrix* matrix, uint32_t tokens);
 
 /* q8gpu_product_device with caller-provided device work space of at least
  * q8gpu_workspace_bytes: a multi-token product of a matrix whose blocks share
- * one scale per row, or of a per-block scale matrix that
- * q8gpu_prepare_matrix_cores has folded, then runs on the int8 matrix cores
- * (same bits). NULL work space = q8gpu_product_device. Returns IRIS_E_RANGE
- * (-5) when it is too small. Asynchronous: it allocates nothing and never
- * changes the matrix. The synchronous q8gpu_product uses its own work
- * space. */
+ * one scale per row, of a per-block scale matrix that
+ * q8gpu_prepare_matrix_cores has folded, or of one whose rows' scales spread
+ * over at most four binary orders, folded or not, then runs on the int8
+ * matrix cores (same bits). NULL work space = q8gpu_product_device. Returns
+ * IRIS_E_RANGE (-5) when it is too small. Asynchronous: it allocates nothing
+ * and never changes the matrix. The synchronous q8gpu_product uses its own
+ * work space. */
 int q8gpu_product_device_ws(const Q8GpuMatrix* matrix, const int32_t* d_activations, uint32_t tokens,
                             int32_t* d_out, void* d_workspace, uint64_t workspace_bytes, void* stream);
 

@@ -28,16 +28,12 @@
 
 #include "detnum_dev.h"
 #include "q8_epilogue.h"
+#include "q8_gemm_common.h"
 #include "q8_internal.h"
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-
-constexpr int PL_MAX = 5;                   // digit planes of an i32
 constexpr uint32_t GM_TT = 4;               // 32-token tiles per workgroup (128 tokens)
-constexpr uint32_t FRAG = 1024;             // bytes of one 32 x 32 operand
 constexpr uint32_t GM_BAND = 8;             // row groups per band of the launch order
 
 // The two workgroup shapes: W waves in a (W/2) x 2 grid over 32 * W rows and
@@ -62,20 +58,6 @@ struct GemmShape {
     static constexpr uint32_t SMEM = SPLIT * RING > OUT ? SPLIT * RING : OUT;
 };
 
-__device__ __forceinline__ uint64_t digits5(int32_t v) {
-    return (uint64_t)((int64_t)v + 0x8080808080LL) ^ 0x8080808080ULL;
-}
-
-__device__ __forceinline__ int limbs_needed(uint64_t d) {
-    return (d >> 32) ? 5 : (d >> 24) ? 4 : (d >> 16) ? 3 : (d >> 8) ? 2 : 1;
-}
-
-__device__ __forceinline__ uint32_t plane_byte4(uint64_t d0, uint64_t d1, uint64_t d2, uint64_t d3, int l) {
-    const int sh = 8 * l;
-    return (uint32_t)((d0 >> sh) & 0xff) | ((uint32_t)((d1 >> sh) & 0xff) << 8) | ((uint32_t)((d2 >> sh) & 0xff) << 16) |
-           ((uint32_t)((d3 >> sh) & 0xff) << 24);
-}
-
 // Per token, one wave each, under the rms_norm prologue only: the token's
 // scale (ops.rs:98-114, rms_norm_scale of the order-free saturating sum of
 // squares) at token_limbs[t].
@@ -97,8 +79,6 @@ __global__ __launch_bounds__(256) void token_prep_kernel(const GemvArgs a) {
         if (lane == 0) a.token_limbs[t] = dn::rms_scale_from_sum(s, K, a.norm_eps);
     }
 }
-
-constexpr uint32_t PLANE_KB = GEMM_PLANE_KB;
 
 __global__ __launch_bounds__(256) void fill_ints_kernel(int32_t* p, uint32_t n, int32_t v) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -155,24 +135,6 @@ __global__ __launch_bounds__(256) void digit_planes_kernel(const GemvArgs a) {
     if (lane == 0) atomicMax(&s_need, need);  // the largest of four: any order
     __syncthreads();
     if (tid == 0) a.token_limbs[M + blockIdx.y * TT + tt] = s_need;
-}
-
-// The digits a workgroup's token tiles tt0 .. tt0 + tg - 1 need: the most
-// any k chunk of them needs, from digit_planes_kernel's counts.
-__device__ __forceinline__ int tiles_limbs(const GemvArgs& a, uint32_t tt0, uint32_t tg, int& s_limbs) {
-    const uint32_t tid = threadIdx.x, TT = (a.tokens + 31) / 32;
-    const uint32_t chunks = (a.w.cols / 32 + PLANE_KB - 1) / PLANE_KB;
-    const int32_t* need = a.token_limbs + a.tokens;
-    if (tid == 0) s_limbs = 1;
-    __syncthreads();
-    for (uint32_t i = tid; i < tg * chunks; i += blockDim.x) {
-        const uint32_t t = tt0 + i % tg;
-        if (t < TT) atomicMax(&s_limbs, need[(i / tg) * TT + t]);
-    }
-    __syncthreads();
-    const int limbs = s_limbs;
-    __syncthreads();
-    return limbs;
 }
 
 template <int N>
@@ -812,6 +774,7 @@ __global__ __launch_bounds__(256, 1) void q8_gemm_fold_kernel(const GemvArgs a) 
 }  // namespace
 
 bool iris_gemm_applies(const GemvArgs& a) {
+    if (iris_skinny_applies(a)) return true;
     if (!a.planes || !a.token_limbs || a.tokens < 2 || a.w.cols % 64 || a.epilogue == EPI_HEAD_SELECT ||
         a.prologue == PRO_NORM_RES_NORM)
         return false;
@@ -844,6 +807,7 @@ int iris_gemm_launch(const GemvArgs& a, hipStream_t stream) {
     }
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return (int)st;
+    if (iris_skinny_applies(a)) return iris_skinny_launch(a, stream);
     if (a.w.scale_mode == Q8_SCALE_F16) {
         // 32-row tiles per workgroup: 4, or 2 for four to six planes (FoldShape::RT).
         const uint32_t rt = a.w.fold_nplanes <= 3 ? 4 : 2;
@@ -893,14 +857,12 @@ int iris_gemm_launch(const GemvArgs& a, hipStream_t stream) {
 int iris_q8_prepare_fold(Q8GpuMatrix* m, hipStream_t stream) {
     static std::mutex lock;  // a matrix is folded once, whichever thread gets there first
     std::lock_guard<std::mutex> guard(lock);
-    if (!m || m->fold_tried || m->scale_mode != Q8_SCALE_F16 || !m->sc16 || m->cols % 64) return 0;
+    if (!m || m->fold_tried || m->scale_mode != Q8_SCALE_F16 || !m->sc16 || !m->fold.shift || m->cols % 64) return 0;
     m->fold_tried = true;
     const size_t plane_bytes = (size_t)m->tiles * m->nb * Q8_TILE_BLOCK_BYTES;
     int* d_need = nullptr;
     int need = 0;
-    hipError_t st = hipMalloc((void**)&m->fold.shift, (size_t)m->tiles * Q8_TILE_ROWS * sizeof(int32_t));
-    if (st == hipSuccess) st = hipMalloc((void**)&d_need, sizeof(int));
-    if (st == hipSuccess) st = hipMemsetAsync(m->fold.shift, 0, (size_t)m->tiles * Q8_TILE_ROWS * sizeof(int32_t), stream);
+    hipError_t st = hipMalloc((void**)&d_need, sizeof(int));
     if (st == hipSuccess) st = hipMemsetAsync(d_need, 0, sizeof(int), stream);
     if (st == hipSuccess) {
         hipLaunchKernelGGL(fold_rows_kernel, dim3((m->rows + 255) / 256), dim3(256), 0, stream, m->qs, m->sc16, m->rows,
@@ -928,7 +890,6 @@ int iris_q8_prepare_fold(Q8GpuMatrix* m, hipStream_t stream) {
         }
     }
     hipFree(m->fold.planes);
-    hipFree(m->fold.shift);
-    m->fold = Q8Folded{};
+    m->fold.planes = nullptr;
     return (int)st;
 }

@@ -877,19 +877,46 @@ __global__ void q8_pack_kernel(const uint8_t* raw, uint32_t rows, uint32_t nb, u
     if (((bits >> 10) & 0x1f) == 0x1f) atomicOr(flags, 1);
 }
 
-// One thread per row: the row's common scale, or flags bit 1 when its blocks
-// differ in value.
-__global__ void q8_row_scale_kernel(const uint16_t* sc16, uint32_t rows, uint32_t nb, int64_t* row_scale,
-                                    int* flags) {
-    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
-    const uint32_t tile = row / Q8_TILE_ROWS, r = row % Q8_TILE_ROWS;
+// One wave per 16-row tile (four blocks of its rows a step, so the scales
+// are read as whole lines): each row's common scale, or flags[0] bit 1 when
+// its blocks differ in value; each row's least exponent shift among its
+// non-zero scales (0 for an all-zero row); and, raised into flags[1], the
+// signed byte digits that a weight of -128 or 127 times the row's largest
+// scale over that shift can need.
+__global__ __launch_bounds__(256) void q8_row_scale_kernel(const uint16_t* sc16, uint32_t tiles, uint32_t nb,
+                                                           int64_t* row_scale, int32_t* row_shift, int* flags) {
+    const uint32_t tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane % Q8_TILE_ROWS;
+    if (tile >= tiles) return;
     const uint16_t* s = sc16 + (size_t)tile * nb * Q8_TILE_ROWS + r;
     const int64_t first = dn::scale_q24(s[0]);
     bool same = true;
-    for (uint32_t b = 1; b < nb; b++) same &= dn::scale_q24(s[(size_t)b * Q8_TILE_ROWS]) == first;
-    row_scale[row] = first;
-    if (!same) atomicOr(flags, 2);
+    int least = 64;
+    int64_t most = 0;
+    for (uint32_t b = lane / Q8_TILE_ROWS; b < nb; b += 4) {
+        const uint32_t bits = s[(size_t)b * Q8_TILE_ROWS], e = (bits >> 10) & 0x1f;
+        const int64_t v = dn::scale_q24(bits);
+        same &= v == first;
+        if (v) least = min(least, e ? (int)e - 1 : 0);
+        most = max(most, v < 0 ? -v : v);
+    }
+    for (int off = 16; off <= 32; off <<= 1) {
+        least = min(least, __shfl_xor(least, off));
+        most = max(most, __shfl_xor(most, off));
+    }
+    if (least == 64) least = 0;
+    if (lane < Q8_TILE_ROWS) {
+        row_scale[tile * Q8_TILE_ROWS + r] = first;
+        row_shift[tile * Q8_TILE_ROWS + r] = least;
+    }
+    const int64_t top = 128 * (most >> least);  // under 2^48
+    int digits = 1;
+    while (digits < 7 && top > 0x7f7f7f7f7f7fLL >> (8 * (6 - digits))) digits++;
+    for (int off = 1; off <= 8; off <<= 1) digits = max(digits, __shfl_xor(digits, off));
+    const bool differ = __any(!same);
+    if (lane == 0) {
+        if (differ) atomicOr(flags, 2);
+        atomicMax(flags + 1, digits);
+    }
 }
 
 }  // namespace
@@ -1043,10 +1070,12 @@ int iris_gemv_launch(const GemvArgs& a, hipStream_t stream) {
 
 int iris_q8_pack_device(const uint8_t* d_raw, Q8GpuMatrix* m, hipStream_t stream, uint32_t interleave_half) {
     int* d_flags = nullptr;
-    int flags = 0;
-    hipError_t st = hipMalloc(&d_flags, sizeof(int));
+    int flags[2] = {0, 0};
+    const size_t shift_bytes = (size_t)m->tiles * Q8_TILE_ROWS * sizeof(int32_t);
+    hipError_t st = hipMalloc(&d_flags, sizeof(flags));
     if (st != hipSuccess) return (int)st;
-    st = hipMemsetAsync(d_flags, 0, sizeof(int), stream);
+    st = hipMemsetAsync(d_flags, 0, sizeof(flags), stream);
+    if (st == hipSuccess) st = hipMalloc((void**)&m->fold.shift, shift_bytes);
     const size_t n = (size_t)m->rows * m->nb;
     if (st == hipSuccess && n) {
         hipLaunchKernelGGL(q8_pack_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, d_raw, m->rows,
@@ -1054,15 +1083,21 @@ int iris_q8_pack_device(const uint8_t* d_raw, Q8GpuMatrix* m, hipStream_t stream
         st = hipGetLastError();
     }
     if (st == hipSuccess && m->rows) {
-        hipLaunchKernelGGL(q8_row_scale_kernel, dim3((m->rows + 255) / 256), dim3(256), 0, stream, m->sc16, m->rows,
-                           m->nb, m->row_scale, d_flags);
+        hipLaunchKernelGGL(q8_row_scale_kernel, dim3((m->tiles + 3) / 4), dim3(256), 0, stream, m->sc16, m->tiles,
+                           m->nb, m->row_scale, m->fold.shift, d_flags);
         st = hipGetLastError();
     }
-    if (st == hipSuccess) st = hipMemcpyAsync(&flags, d_flags, sizeof(int), hipMemcpyDeviceToHost, stream);
+    if (st == hipSuccess) st = hipMemcpyAsync(flags, d_flags, sizeof(flags), hipMemcpyDeviceToHost, stream);
     if (st == hipSuccess) st = hipStreamSynchronize(stream);
     hipFree(d_flags);
     if (st != hipSuccess) return (int)st;
-    if (flags & 1) return IRIS_E_SCALE;
-    m->scale_mode = (flags & 2) ? Q8_SCALE_F16 : Q8_SCALE_ROW;
+    if (flags[0] & 1) return IRIS_E_SCALE;
+    m->scale_mode = (flags[0] & 2) ? Q8_SCALE_F16 : Q8_SCALE_ROW;
+    if (m->scale_mode == Q8_SCALE_F16) {
+        m->digits_bound = (uint32_t)flags[1];
+    } else {
+        hipFree(m->fold.shift);
+        m->fold.shift = nullptr;
+    }
     return 0;
 }

@@ -40,7 +40,7 @@ constexpr int Q8_TILE_BLOCK_BYTES = 512;
 struct Q8Folded {
     int8_t* planes;    // [planes][tiles][nb][512]
     int32_t* shift;    // [tiles * 16]
-    uint32_t nplanes;  // 0 = not prepared
+    uint32_t nplanes;  // 0 = planes not built
 };
 
 // Weight digit planes of a folded matrix, at most: the widest spread of a
@@ -57,7 +57,12 @@ struct Q8GpuMatrix {
     int64_t* sc64;
     int64_t* row_scale;
     uint64_t device_bytes;
+    // Per-block f16 scales: fold.shift (R per row) and a bound on the digits
+    // of the row's w' (from the scales alone, for weights of either extreme)
+    // come with the upload; the planes only with iris_q8_prepare_fold. (The
+    // reported device_bytes count the shifts with the planes.)
     Q8Folded fold;
+    uint32_t digits_bound;
     bool fold_tried;  // the folding was attempted (prepared or refused)
 };
 
@@ -72,11 +77,13 @@ struct Q8View {
     const int8_t* fold_planes;
     const int32_t* fold_shift;
     uint32_t fold_nplanes;
+    uint32_t digits_bound;
 };
 
 inline Q8View q8_view(const Q8GpuMatrix* m) {
     return Q8View{m->qs,   m->sc16,       m->sc64,       m->row_scale,      m->rows,        m->cols,
-                  m->nb,   m->tiles,      m->scale_mode, m->fold.planes,    m->fold.shift,  m->fold.nplanes};
+                  m->nb,   m->tiles,      m->scale_mode, m->fold.planes,    m->fold.shift,  m->fold.nplanes,
+                  m->digits_bound};
 }
 
 // Builds m's folded planes (once; per-block scale matrices only) so that

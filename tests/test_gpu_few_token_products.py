@@ -1,0 +1,38 @@
+"""GPU parity of the products of few tokens (16 x 16 and 32 x 32 tiles, the
+waves sharing one tile's k steps) against the oracle, every output exact."""
+import numpy as np
+import pytest
+
+from iris_amd import native, synth
+from iris_amd.tensor import Q8Matrix
+from oracle import cpu
+from test_gpu_q8_product import per_block_matrix, product_ws, rand_activations
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    native.check(native.lib().q8gpu_init(), "q8gpu_init")
+
+
+# Token counts at the edges of both tile shapes and of their dispatch; rows
+# that leave the last 16-row tile partial or a 32-row tile half empty; one k
+# step, fewer steps than waves, and step counts that leave waves uneven.
+@pytest.mark.parametrize("tokens,rows,cols", [(2, 1, 64), (16, 17, 64), (13, 200, 4160), (17, 16, 128), (32, 33, 576),
+                                              (33, 250, 4160), (64, 144, 1088), (65, 48, 192), (16, 4100, 256),
+                                              (31, 48, 14336)])
+@pytest.mark.parametrize("kind", ["row", "unit", "tiny", "same", "spread4"])
+def test_few_token_products(tokens, rows, cols, kind):
+    print(f"{kind} tokens {tokens} rows {rows} cols {cols}", flush=True)
+    rng = np.random.default_rng(tokens * 31 + rows + cols)
+    if kind == "row":
+        raw = synth.q8_matrix(synth.tensor_seed(19, rows), rows, cols, synth.scale_base_for(cols), True)
+    else:
+        raw = per_block_matrix(rng, rows, cols, kind)
+    m = Q8Matrix.from_bytes(raw, rows, cols)
+    for bits in (7, 16, 22, 32):  # one to five activation digits
+        x = rand_activations(rng, tokens, cols, bits)
+        if bits < 32:
+            x = np.clip(x, -(1 << (bits - 1)), (1 << (bits - 1)) - 1).astype(np.int32)
+        assert np.array_equal(product_ws(m, x), cpu.linear_q8(x, raw))
