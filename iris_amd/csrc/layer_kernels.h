@@ -172,4 +172,8 @@ int iris_ple_prepare_launch(const PleArgs& a, uint32_t segments, uint32_t rows, 
 // `rows` positions from *d_pos and j < half: out[row][j][2].
 int iris_rope_table_launch(const int64_t* inv_freq, uint32_t half, const int32_t* d_pos, uint32_t rows, int64_t* out,
                            hipStream_t stream);
+// K cache positions pos0..pos0 + count as rows of kvw values (out), or rows
+// into the cache: kv_rows.hip.
+int iris_kv_rows_launch(bool out, int32_t* cache, uint32_t stride, uint32_t pos0, uint32_t count, uint32_t kvw,
+                        int32_t* rows, hipStream_t stream);
 int iris_rope_ladder_launch(int64_t base, uint32_t freq_base_dim, uint32_t half, int64_t* out, hipStream_t stream);

@@ -1202,6 +1202,7 @@ void iris_session_free(IrisSession* s) {
     hipFree(s->attn_planes.kv_limbs);
     hipFree(s->attn_planes.e_store);
     hipFree(s->rope_sc);
+    hipFree(s->kv_stage);
     hipFree(s->ckpt_dev);
     if (s->ckpt_host) hipHostFree(s->ckpt_host);
     for (auto e : s->ckpt_events)
@@ -1416,8 +1417,24 @@ static int layer_stage_run(IrisSession* s, uint32_t layer, const int32_t* in_row
     return (int)hipStreamSynchronize(st);
 }
 
+// The device staging for K rows: at most 4 Mi ints (16 MB), so longer blocks
+// go over in chunks of that many positions.
+static int ensure_kv_stage(IrisSession* s, size_t kvw, uint32_t count, uint32_t* chunk) {
+    const size_t most = std::max<size_t>(kvw, (size_t)4 << 20);
+    *chunk = (uint32_t)std::min<size_t>(count, most / kvw);
+    const size_t need = (size_t)*chunk * kvw;
+    if (need <= s->kv_stage_cap) return 0;
+    RT_CHECK(hipFree(s->kv_stage));
+    s->kv_stage = nullptr;
+    s->kv_stage_cap = 0;
+    RT_CHECK(hipMalloc((void**)&s->kv_stage, need * 4));
+    s->kv_stage_cap = need;
+    return 0;
+}
+
 // Carried keys into a layer's cache: one kv row of k and of v per position,
-// the K side transposed into the cache's [kv_rows][k_pos_stride] layout.
+// the K side transposed on the device into the cache's [kv_rows][k_pos_stride]
+// layout.
 int iris_session_write_kv(IrisSession* s, uint32_t layer, uint32_t pos0, uint32_t count, const int32_t* k,
                           const int32_t* v) {
     if (!s || (count && (!k || !v))) return IRIS_E_INVALID;
@@ -1426,25 +1443,24 @@ int iris_session_write_kv(IrisSession* s, uint32_t layer, uint32_t pos0, uint32_
     if ((uint64_t)pos0 + count > s->max_positions) return IRIS_E_RANGE;
     if (count == 0) return 0;
     const size_t kvw = s->model->layers[layer].kv_rows;
-    std::vector<int32_t> kt;
-    try {
-        kt.resize(kvw * count);
-    } catch (...) {
-        return IRIS_E_NOMEM;
+    uint32_t chunk = 0;
+    RT_CHECK(ensure_kv_stage(s, kvw, count, &chunk));
+    for (uint32_t p = 0; p < count; p += chunk) {
+        const uint32_t n = std::min(chunk, count - p);
+        RT_CHECK(hipMemcpyAsync(s->kv_stage, k + p * kvw, n * kvw * 4, hipMemcpyHostToDevice, s->stream));
+        RT_CHECK(iris_kv_rows_launch(false, s->k_cache[layer], s->k_pos_stride, pos0 + p, n, (uint32_t)kvw, s->kv_stage,
+                                     s->stream));
     }
-    for (size_t p = 0; p < count; p++)
-        for (size_t c = 0; c < kvw; c++) kt[c * count + p] = k[p * kvw + c];
+    RT_CHECK(hipMemcpyAsync(s->v_cache[layer] + (size_t)pos0 * kvw, v, (size_t)count * kvw * 4, hipMemcpyHostToDevice,
+                            s->stream));
     RT_CHECK(hipStreamSynchronize(s->stream));
-    RT_CHECK(hipMemcpy2D(s->k_cache[layer] + pos0, (size_t)s->k_pos_stride * 4, kt.data(), (size_t)count * 4,
-                         (size_t)count * 4, kvw, hipMemcpyHostToDevice));
-    RT_CHECK(hipMemcpy(s->v_cache[layer] + (size_t)pos0 * kvw, v, (size_t)count * kvw * 4, hipMemcpyHostToDevice));
     cover(s, layer, pos0, count);
     return 0;
 }
 
-// The K cache is transposed ([kv_rows][k_pos_stride]): the block of the
-// asked positions comes over as kv_rows strided runs and is transposed into
-// position rows on the host; V rows are already position rows.
+// The K cache is transposed ([kv_rows][k_pos_stride]): the asked positions
+// are transposed into rows on the device and come over as one run; V rows
+// are already position rows.
 int iris_session_read_kv(IrisSession* s, uint32_t layer, uint32_t pos0, uint32_t count, int32_t* k_out,
                          int32_t* v_out) {
     if (!s || (count && (!k_out || !v_out))) return IRIS_E_INVALID;
@@ -1453,20 +1469,17 @@ int iris_session_read_kv(IrisSession* s, uint32_t layer, uint32_t pos0, uint32_t
     if ((uint64_t)pos0 + count > s->max_positions) return IRIS_E_RANGE;
     if (count == 0) return 0;
     const size_t kvw = s->model->layers[layer].kv_rows;
-    std::vector<int32_t> kt;
-    try {
-        kt.resize(kvw * count);
-    } catch (...) {
-        return IRIS_E_NOMEM;
+    uint32_t chunk = 0;
+    RT_CHECK(ensure_kv_stage(s, kvw, count, &chunk));
+    for (uint32_t p = 0; p < count; p += chunk) {
+        const uint32_t n = std::min(chunk, count - p);
+        RT_CHECK(iris_kv_rows_launch(true, s->k_cache[layer], s->k_pos_stride, pos0 + p, n, (uint32_t)kvw, s->kv_stage,
+                                     s->stream));
+        RT_CHECK(hipMemcpyAsync(k_out + p * kvw, s->kv_stage, n * kvw * 4, hipMemcpyDeviceToHost, s->stream));
     }
-    RT_CHECK(hipStreamSynchronize(s->stream));
-    RT_CHECK(hipMemcpy2D(kt.data(), (size_t)count * 4, s->k_cache[layer] + pos0, (size_t)s->k_pos_stride * 4,
-                         (size_t)count * 4, kvw, hipMemcpyDeviceToHost));
-    RT_CHECK(hipMemcpy(v_out, s->v_cache[layer] + (size_t)pos0 * kvw, (size_t)count * kvw * 4,
-                       hipMemcpyDeviceToHost));
-    for (size_t c = 0; c < kvw; c++)
-        for (size_t p = 0; p < count; p++) k_out[p * kvw + c] = kt[c * count + p];
-    return 0;
+    RT_CHECK(hipMemcpyAsync(v_out, s->v_cache[layer] + (size_t)pos0 * kvw, (size_t)count * kvw * 4,
+                            hipMemcpyDeviceToHost, s->stream));
+    return (int)hipStreamSynchronize(s->stream);
 }
 
 int iris_kernel_tracer_loaded(void) { return kernel_tracer_loaded() ? 1 : 0; }

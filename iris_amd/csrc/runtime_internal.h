@@ -124,6 +124,10 @@ struct IrisSession {
     int64_t* rope_sc = nullptr;      // mistral-dense: [max_rows][head_dim/2][sin, cos] of the pass's positions
     // multi-row attention digit planes (null for single-row sessions)
     AttnPlanes attn_planes{};
+    // K rows on their way to or from the host (kv_stage_chunk positions at
+    // most), made on the first iris_session_read_kv / write_kv
+    int32_t* kv_stage = nullptr;
+    size_t kv_stage_cap = 0;  // ints
     // per-layer checkpoint staging, made on the first checkpointing pass
     int32_t* ckpt_dev = nullptr;              // [layers][max_rows][hidden]
     uint8_t* ckpt_host = nullptr;             // pinned, same shape
