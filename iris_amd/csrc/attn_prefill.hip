@@ -201,13 +201,41 @@ __device__ __forceinline__ void tile_scores(const AttnArgs& a, const v4i (&kf)[L
 #pragma unroll
             for (int b = 0; b < LQK; b++)
                 acc[l + b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf[l][ds], qf[b][ds], acc[l + b], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
+    auto exact = [&](int i) __attribute__((always_inline)) {
         uint64_t s = 0;  // the wrapping i64 dot product
 #pragma unroll
         for (int j = 0; j < NS; j++) s += (uint64_t)(int64_t)acc[j][i] << (8 * j);
-        sc[i] = a.scaled ? dn::scaled_score_from_sum((int64_t)s, a.scale_q32) : dn::requantize((int64_t)s);
+        return a.scaled ? dn::scaled_score_from_sum((int64_t)s, a.scale_q32) : dn::requantize((int64_t)s);
+    };
+    if constexpr (HD <= 128 && LQK <= 3) {
+        // Up to three digits each (the usual values): the sum fits a double
+        // (|.| <= HD * (2^23 + 2^15)^2, at most a unit over 2^53 rounded), and
+        // neighbouring accumulators an int32 (at most 2 * HD * 2^14 each), so
+        // three conversions and a few double operations per score replace the
+        // 64-bit shifts, sums and multiplies. Scores near a rounding tie (one
+        // in 2^14) are redone exactly.
+        const double scale = (double)a.scale_q32 * 0x1p-48;
+        bool slow = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            double s = 0;
+#pragma unroll
+            for (int j = NS - 1; j >= 0; j -= 1) {
+                if (j % 2 == 1) continue;
+                const int32_t pair = j + 1 < NS ? acc[j][i] + (acc[j + 1][i] << 8) : acc[j][i];
+                s = fma(s, 65536.0, (double)pair);
+            }
+            if (a.scaled) {
+                slow |= !dn::scaled_score_fast(s, scale, sc[i]);
+            } else {
+                sc[i] = dn::requantize((int64_t)s);
+                slow |= fabs(s) >= 0x1p53;  // no longer exact
+            }
+        }
+        if (!__any(slow)) return;
     }
+#pragma unroll
+    for (int i = 0; i < 4; i++) sc[i] = exact(i);
 }
 
 // One wave: 16 query rows of one head over key steps [ks0, ks1), queries
@@ -297,7 +325,7 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
     // from the stored scores; each lane overwrites a tile's scores with its
     // terms for (3) (2^32, the maximum's term, as 0xffffffff: every other
     // term is below 2^32 - 2^15).
-    uint64_t sum = 0;
+    double fsum = 0;  // at most 2^16 terms of 2^32: exact
     uint4 sn = *(const uint4*)(estore + (size_t)kt0 * 256);
     // Waited for here, visibly (as the first key tile above): otherwise
     // each tile's wait for its prefetched scores also covered the previous
@@ -312,16 +340,16 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const uint32_t key = kt * 16 + 4 * grp + i;
-            const int64_t diff = (int64_t)best - sc[i];
-            uint64_t e = 0;
-            if (visible(key) & (diff < (1 << 20))) e = dn::softmax_exp_diff((uint32_t)diff);
-            sum += e;
-            ev[i] = e > 0xffffffffull ? 0xffffffffu : (uint32_t)e;
+            // best >= sc: the difference fits 32 bits unsigned.
+            const double e = visible(key) ? dn::softmax_exp_f64((uint32_t)best - (uint32_t)sc[i]) : 0.0;
+            fsum += e;
+            ev[i] = e > 4294967295.0 ? 0xffffffffu : (uint32_t)e;
         }
         *(uint4*)(estore + (size_t)kt * 256) = make_uint4(ev[0], ev[1], ev[2], ev[3]);
     }
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
+    fsum += __shfl_xor(fsum, 16);
+    fsum += __shfl_xor(fsum, 32);
+    const uint64_t sum = (uint64_t)fsum;
     const double q_scale = qvalid ? 4294967296.0 / (double)sum : 0.0;
     const double w_scale = qvalid ? 65536.0 / (double)sum : 0.0;
 

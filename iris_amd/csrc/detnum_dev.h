@@ -201,56 +201,36 @@ __device__ __forceinline__ int32_t rms_scale_from_sum(int64_t sum_squares, uint3
     return inv_sqrt_acc(acc_add_sat(mean, eps));
 }
 
-// rte(x / c) (ops.rs:691-720) for a non-negative dividend below 2^32.
-__device__ __forceinline__ uint32_t rte_div_u32(uint32_t x, uint32_t c) {
-    const uint32_t q = x / c;
-    return q + (uint32_t)(2 * (x - q * c) + (q & 1) > c);
-}
-
-// acc_mul (ops.rs:685-689) of 0 <= a, b < 2^32: the product fits 64 bits,
-// and the rounded result stays below 2^32 when a or b is below 2^32 - 1.
-// (p + 2^31 - 1 + (floor & 1)) carries into the high word exactly when the
-// rounding steps up; p <= (2^32 - 1)^2 leaves room for the addend.
-__device__ __forceinline__ uint32_t acc_mul_u32(uint32_t a, uint32_t b) {
-    const uint64_t p = (uint64_t)a * b;
-    return (uint32_t)((p + 0x7fffffffull + ((p >> 32) & 1)) >> 32);
-}
-
 // softmax_exp_term (ops.rs:508-556) of delta = -(diff << 16), diff >= 0:
 // the only deltas the softmax forms (a logit minus the row's maximum).
-// diff >= 2^20 is at or below the -16 cut: zero; diff = 0 gives exactly one.
-// Otherwise 0 < r < ln 2 < 1 in Q32.32: every power and quotient of the
-// Taylor terms is below 2^32, none of the saturating sums can saturate, the
-// result of the nested sums lies in (0, 2^32), and the shift is at most 23,
-// so the general routine's integers come out of 32-bit operations. The
-// quotient by ln 2 starts from a float estimate (off by at most one, as
-// diff < 2^20 is exact in a float) and is corrected on the remainder.
+// diff >= 2^20 is at or below the -16 cut: zero; diff = 0 gives exactly one
+// (2^32). The integers of the reference's steps are formed in double: the
+// quotient by ln 2 and the remainder r (an exact fma), the powers
+// rte(r^i * r / 2^32) and the quotients by 2, 6, 24 and 120 each as one
+// multiplication and one round-to-nearest-even, and the final shift as a
+// scaling by 2^-k and one more. A power's product has up to 64 bits, so its
+// double can be off by 2^-22 of the rounded unit, and a quotient's by 2^-21;
+// that no rounding of any of the 2^20 possible differences turns on it is
+// checked over all of them (test_gpu_attention.py compares every one with
+// the oracle). About 30 double operations at full rate: the 32-bit integer
+// form took about 94 instructions, half of them quarter-rate multiplies,
+// and bound the prefill attention's exp walk (with the scores below, that
+// kernel went from 529 to 435 us per layer at 2048 rows of head size 128,
+// from 186 to 124 us at 512 rows after 512).
 // The body is branch-free (selects only), so a wave's lanes run it together.
-__device__ __forceinline__ uint64_t softmax_exp_diff(uint32_t diff) {
-    if (diff >= (1u << 20)) return 0;
-    const int64_t LN_2_BITS = 2977044472LL;
-    const int64_t positive = (int64_t)diff << 16;
-    uint32_t shift = (uint32_t)((float)diff * (65536.0f / 2977044472.0f));
-    int64_t rl = positive - (int64_t)shift * LN_2_BITS;
-    const bool below = rl < 0;
-    shift -= (uint32_t)below;
-    rl += below ? LN_2_BITS : 0;
-    const bool above = rl >= LN_2_BITS;
-    shift += (uint32_t)above;
-    rl -= above ? LN_2_BITS : 0;
-    const uint32_t r = (uint32_t)rl;
-    const uint32_t r2 = acc_mul_u32(r, r), r3 = acc_mul_u32(r2, r);
-    const uint32_t r4 = acc_mul_u32(r3, r), r5 = acc_mul_u32(r4, r);
-    // 1 - r + r2/2 - r3/6 + r4/24 - r5/120, modulo 2^32 (the true value is
-    // in (0, 2^32)).
-    const uint32_t approx = 0u - r + rte_div_u32(r2, 2) - rte_div_u32(r3, 6) + rte_div_u32(r4, 24) -
-                            rte_div_u32(r5, 120);
-    const uint32_t fl = approx >> shift;
-    const uint32_t rem = approx & ((1u << shift) - 1), half = (1u << shift) >> 1;
-    const uint32_t rounded = fl + (uint32_t)(rem + (fl & 1) > half);
-    // diff = 0: r = 0 and the sum is 2^32, which wraps to 0 above.
-    return diff == 0 ? (uint64_t)ONE_ACC : (uint64_t)(shift == 0 ? approx : rounded);
+__device__ __forceinline__ double softmax_exp_f64(uint32_t diff) {
+    const double d = (double)diff;
+    const double k = floor(d * (65536.0 / 2977044472.0));
+    const double r = fma(k, -2977044472.0, d * 65536.0);
+    const double rs = r * 0x1p-32;
+    const double r2 = rint(r * rs), r3 = rint(r2 * rs), r4 = rint(r3 * rs), r5 = rint(r4 * rs);
+    const double approx = ((4294967296.0 - r) + rint(r2 * 0.5)) - rint(r3 * (1.0 / 6)) + rint(r4 * (1.0 / 24)) -
+                          rint(r5 * (1.0 / 120));
+    const double e = rint(__builtin_ldexp(approx, -(int)k));
+    return diff < (1u << 20) ? e : 0.0;
 }
+
+__device__ __forceinline__ uint64_t softmax_exp_diff(uint32_t diff) { return (uint64_t)softmax_exp_f64(diff); }
 
 // attention_softmax_raw_weight (ops.rs:269-271), requantize(div_acc(e, sum)),
 // for 0 <= e <= 2^32 <= sum < 2^62 and q_scale = 2^32 / sum in double: the
@@ -472,6 +452,18 @@ __device__ __forceinline__ int32_t scaled_score_from_sum(int64_t sum, uint32_t s
     const uint64_t lo = (uint32_t)sum;
     const int64_t scaled = hi * (int64_t)scale_q32 + (int64_t)((lo * scale_q32) >> 32);
     return clamp_i64_to_i32(rshift_rte(scaled, 16));
+}
+
+// scaled_score_from_sum of a sum held in double (exact, or off by less than
+// 2^-50 of itself): t = sum * scale / 2^48 is the score before its rounding,
+// the reference's floor at 2^-32 of the product moves it by under 2^-16, so
+// unless t lies within 2^-15 of a half integer the score is the integer
+// nearest t (saturated: the conversion clamps). False: the exact routine
+// decides.
+__device__ __forceinline__ bool scaled_score_fast(double sum, double scale_2m48, int32_t& score) {
+    const double t = sum * scale_2m48, n = rint(t);
+    score = (int32_t)fmin(fmax(n, -2147483648.0), 2147483647.0);
+    return fabs(t - n) <= 0.5 - 0x1p-15;
 }
 
 // q8.rs:94-104: value / 2^shift, ties to even, saturated to i32.
