@@ -1,0 +1,7 @@
+// The tiled multi-token products' launches, planes and counts made.
+#pragma once
+
+#include "q8_internal.h"
+
+int iris_gemm_row_launch(const GemvArgs& a, hipStream_t stream);
+int iris_gemm_fold_launch(const GemvArgs& a, hipStream_t stream);
