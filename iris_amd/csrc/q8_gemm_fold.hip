@@ -128,38 +128,38 @@ __device__ __forceinline__ void fold_mainloop(const GemvArgs& a, int8_t* smem, u
                                               v16i (&acc)[G::RI][G::NS]) {
     constexpr uint32_t TTWG = G::TTWG, RT = G::RT, CHUNKS = G::CHUNKS, PER_WAVE = G::PER_WAVE;
     constexpr uint32_t STAGES = G::STAGES, STAGE = G::STAGE;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wr = wave % G::WR, wt = wave / G::WR;
     const Q8View& w = a.w;
     const uint32_t KS = w.cols / 64, KB = w.cols / 32, TT = (a.tokens + 31) / 32;
     const size_t lstride = (size_t)TT * KB * FRAG;
     const size_t pstride = (size_t)w.tiles * w.nb * Q8_TILE_BLOCK_BYTES;
-    // Wave w copies chunks w, w + W, ...: weight-plane operands (1 KB of the
-    // tile layout per k step) first, then digit-plane operands (2 KB).
+    // Wave w copies chunks w, w + W, ...: the first WCH are weight-plane
+    // operands (advancing 1 KB of the tile layout per k step), the rest
+    // digit-plane operands (2 KB).
+    constexpr uint32_t WCH = 2 * RT * WP / G::WAVES;
+    static_assert(WCH * G::WAVES == 2 * RT * WP, "whole chunks per wave");
     const int8_t* src[PER_WAVE];
-    uint32_t step[PER_WAVE];
+    uint32_t off[WCH];
 #pragma unroll
     for (uint32_t i = 0; i < PER_WAVE; i++) {
-        const uint32_t c0 = wave + G::WAVES * i, c = c0 < CHUNKS ? c0 : 0;
-        if (c < 2 * RT * WP) {
-            const uint32_t p = c / (2 * RT), cw = c % (2 * RT), rr = lane & 31, h = lane >> 5, sub = cw & 1;
-            const uint32_t tile16 = min(2 * (rt0 + cw / 2) + rr / 16, w.tiles - 1);
-            src[i] = w.fold_planes + p * pstride + ((size_t)tile16 * w.nb + sub) * Q8_TILE_BLOCK_BYTES + h * 256 +
-                     (rr % 16) * 16;
-            step[i] = FRAG;
+        const uint32_t c = min(wave + G::WAVES * i, CHUNKS - 1);
+        if (i < WCH) {
+            const uint32_t p = c / (2 * RT), cw = c % (2 * RT);
+            src[i] = weight_operand(w, w.fold_planes + p * pstride, rt0 + cw / 2, cw & 1, lane, off[i]);
         } else {
             const uint32_t b = c - 2 * RT * WP, sub = b & 1, rest = b >> 1, l = rest / TTWG;
             const uint32_t tile = min(tt0 + rest % TTWG, TT - 1);
-            src[i] = a.planes + l * lstride + ((size_t)tile * KB + sub) * FRAG + lane * 16;
-            step[i] = 2 * FRAG;
+            src[i] = a.planes + l * lstride + ((size_t)tile * KB + sub) * FRAG;
         }
     }
-    const uint32_t ring = lds_offset(smem);
+    const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset(smem));
     auto issue = [&](uint32_t ks) {
         const uint32_t base = ring + (ks % STAGES) * STAGE;
 #pragma unroll
         for (uint32_t i = 0; i < PER_WAVE; i++)
-            copy_to_lds16(src[i] + (size_t)ks * step[i], base + (wave + G::WAVES * i) * FRAG);
+            copy_to_lds16(src[i] + (size_t)ks * (i < WCH ? FRAG : 2 * FRAG), i < WCH ? off[i] : lane * 16,
+                          base + (wave + G::WAVES * i) * FRAG);
     };
 #pragma unroll
     for (uint32_t s = 0; s < STAGES - 1; s++)
@@ -276,7 +276,12 @@ int iris_gemm_fold_launch(const GemvArgs& a, hipStream_t stream) {
     const uint32_t TT = (a.tokens + 31) / 32, cus = (uint32_t)iris_device_cus();
     const uint32_t rg = (a.w.tiles + 7) / 8, n4 = rg * ((TT + 3) / 4), n2 = rg * ((TT + 1) / 2);
     const uint32_t n64 = (a.w.tiles + 3) / 4 * ((TT + 1) / 2);
-    const bool wide = 2 * ((n4 + cus - 1) / cus) <= (n2 + cus - 1) / cus;
+    // A 128-token workgroup takes about 8/5 of a 64-token one's time. us per
+    // product, preparation included, 128 / 64 tokens, rows x K:
+    //   2048 tokens  28672 x 4096  1637 / 1923    4096 x 14336  841 / 959
+    //    512 tokens  28672 x 4096   455 / 514     4096 x 14336  327 / 245
+    //    128 tokens  28672 x 4096   141 / 158     512 tokens, 4096 x 4096  104 / 78
+    const bool wide = 8 * ((n4 + cus - 1) / cus) <= 5 * ((n2 + cus - 1) / cus);
     switch (a.w.fold_nplanes) {
         case 1: hipLaunchKernelGGL((q8_gemm_fold_kernel<1, 4, 4, 2>), dim3(n2), dim3(256), 0, stream, a); break;
         case 2: hipLaunchKernelGGL((q8_gemm_fold_kernel<2, 4, 4, 2>), dim3(n2), dim3(256), 0, stream, a); break;

@@ -38,7 +38,7 @@ struct GemmShape {
 // where two tiles against two took 8. A stage holds, for its two 32-wide k blocks s, the
 // weight operand of tile r at chunk 2r + s and the plane-l operand of token
 // tile j at 2RT + 2(l * TTWG + j) + s (padded to a whole number of chunks
-// per wave with copies of chunk 0). Operands past the last tile are clamped
+// per wave with copies of the last). Operands past the last tile are clamped
 // onto it (read, never stored).
 template <class G, int LG, int RI, bool DEEP = false>
 __device__ __forceinline__ void gemm_mainloop(const GemvArgs& a, int8_t* smem, uint32_t rt0, uint32_t tt0,
@@ -60,9 +60,9 @@ __device__ __forceinline__ void gemm_mainloop(const GemvArgs& a, int8_t* smem, u
     static_assert(GM_STAGES * GM_STAGE <= G::RING, "ring layout");
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     // The wave within its k group, the group's ring and k steps [ks0, ks1).
-    // The k group through readfirstlane: uniform, so the k loop's control
-    // stays in scalar registers.
-    const uint32_t half = __builtin_amdgcn_readfirstlane((tid >> 6) / G::WAVES), wave = (tid >> 6) % G::WAVES;
+    // Through readfirstlane: uniform, so the k loop's control and the copies'
+    // addresses stay in scalar registers.
+    const uint32_t id = __builtin_amdgcn_readfirstlane(tid >> 6), half = id / G::WAVES, wave = id % G::WAVES;
     const uint32_t wr = wave % WR, wt = wave / WR;
     const Q8View& w = a.w;
     const uint32_t KS = w.cols / 64, KB = w.cols / 32, TT = (a.tokens + 31) / 32;
@@ -74,27 +74,25 @@ __device__ __forceinline__ void gemm_mainloop(const GemvArgs& a, int8_t* smem, u
     // (advancing 1 KB of the tile layout per k step), the rest plane
     // operands (advancing 2 KB).
     const int8_t* src[PER_WAVE];
-    uint32_t step[PER_WAVE];
+    uint32_t off[2];
 #pragma unroll
     for (uint32_t i = 0; i < PER_WAVE; i++) {
-        const uint32_t c0 = wave + G::WAVES * i, c = c0 < CHUNKS ? c0 : 0;
-        step[i] = c < 2 * GM_RT ? FRAG : 2 * FRAG;
-        if (c < 2 * GM_RT) {
-            const uint32_t r = lane & 31, h = lane >> 5, sub = c & 1;
-            const uint32_t tile16 = min(2 * (rt0 + c / 2) + r / 16, w.tiles - 1);
-            src[i] = (const int8_t*)w.qs + ((size_t)tile16 * w.nb + sub) * Q8_TILE_BLOCK_BYTES + h * 256 + (r % 16) * 16;
+        const uint32_t c = min(wave + G::WAVES * i, CHUNKS - 1);
+        if (i < 2) {
+            src[i] = weight_operand(w, (const int8_t*)w.qs, rt0 + c / 2, c & 1, lane, off[i]);
         } else {
             const uint32_t b = c - 2 * GM_RT, sub = b & 1, rest = b >> 1, l = rest / TTWG;
             const uint32_t tile = min(tt0 + rest % TTWG, TT - 1);
-            src[i] = a.planes + l * lstride + ((size_t)tile * KB + sub) * FRAG + lane * 16;
+            src[i] = a.planes + l * lstride + ((size_t)tile * KB + sub) * FRAG;
         }
     }
-    const uint32_t ring = lds_offset(smem);
+    const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset(smem));
     auto issue = [&](uint32_t ks) {
         const uint32_t base = ring + (ks % GM_STAGES) * GM_STAGE;
 #pragma unroll
         for (uint32_t i = 0; i < PER_WAVE; i++)
-            copy_to_lds16(src[i] + (size_t)ks * step[i], base + (wave + G::WAVES * i) * FRAG);
+            copy_to_lds16(src[i] + (size_t)ks * (i < 2 ? FRAG : 2 * FRAG), i < 2 ? off[i] : lane * 16,
+                          base + (wave + G::WAVES * i) * FRAG);
     };
 
 #pragma unroll
@@ -262,27 +260,31 @@ __global__ __launch_bounds__(64 * W * SPLIT, 1) void q8_gemm_row_kernel(const Ge
 
 int iris_gemm_row_launch(const GemvArgs& a, hipStream_t stream) {
     const uint32_t TT = (a.tokens + 31) / 32;
-    // Two waves per SIMD and 256 rows x 128 tokens when that still gives
-    // every CU a workgroup in at most half the rounds of the 128-row shape
-    // (whose workgroups do half the work: q/k/v at 2048 tokens, 384 of the
-    // larger against 768 of the smaller, 2048-row pass 69.35 -> 69.17 ms),
-    // else one wave per SIMD and 128 rows, with 64
-    // tokens when the rounds of workgroups that gives cost less: a 64-token
-    // workgroup takes about 2/3 of a 128-token one's time (M=512, K=N=4096:
-    // 256 of them 60.6 us, 128 of the larger 92.1 us).
+    // The shape whose rounds of workgroups cost least: 256 rows x 128 tokens
+    // with two waves per SIMD, or 128 x 128 or 128 x 64 with the k steps
+    // split between two wave groups. A round of them takes about 11 : 7 : 4
+    // (82, 53 and 30 us at K = 4096 in a full chip). us per product,
+    // preparation included, 256 x 128 / 128 x 128 / 128 x 64, rows x K:
+    //   2048 tokens  28672 x 4096   639 / 736 / 822    6144 x 4096   178 / 175 / 194
+    //   1024 tokens  4096 x 14336   260 / 184 / 214    6144 x 4096    96 / 110 / 104
+    //    512 tokens  28672 x 4096   182 / 212 / 215    4096 x 14336  233 / 142 / 106
+    //    256 tokens  28672 x 4096    95 / 110 / 123    6144 x 4096    78 /  54 /  37
+    //    777 tokens  20000 x 4096   248 / 254 / 245
     const uint32_t n_tg = (TT + GM_TT - 1) / GM_TT, n_tg2 = (TT + 1) / 2;
     const uint32_t cus = (uint32_t)iris_device_cus();
     const uint32_t n8 = (a.w.tiles + 15) / 16 * n_tg, n4 = (a.w.tiles + 7) / 8 * n_tg;
     const uint32_t n42 = (a.w.tiles + 7) / 8 * n_tg2;
-    const uint32_t rounds8 = (n8 + cus - 1) / cus, rounds4 = (n4 + cus - 1) / cus, rounds2 = (n42 + cus - 1) / cus;
-    // The four-wave shapes split the k steps between two wave groups when
-    // there is an even number of them (both groups' barriers pair up).
+    const uint32_t cost8 = 11 * ((n8 + cus - 1) / cus), cost4 = 7 * ((n4 + cus - 1) / cus);
+    const uint32_t cost2 = 4 * ((n42 + cus - 1) / cus);
+    // The k steps are split only when there is an even number of them (both
+    // groups' barriers pair up); else the 128-row shapes have one wave per
+    // SIMD and serve launches that leave CUs without a 256-row workgroup.
     const bool split = (a.w.cols / 64) % 2 == 0;
     // Deeper rings for long rows (at least 64 k steps per wave group).
     const bool deep = a.w.cols >= 8192;
-    if (n8 >= cus && (2 * rounds8 <= rounds4 || !split))
+    if (split ? cost8 <= (cost4 < cost2 ? cost4 : cost2) : n8 >= cus)
         hipLaunchKernelGGL((q8_gemm_row_kernel<8, 4>), dim3(n8), dim3(512), 0, stream, a);
-    else if (n42 != n4 && 2 * rounds2 <= 3 * rounds4) {
+    else if (n42 != n4 && cost2 <= cost4) {
         if (split && deep) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2, 2, true>), dim3(n42), dim3(512), 0, stream, a);
         else if (split) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2, 2>), dim3(n42), dim3(512), 0, stream, a);
         else hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2>), dim3(n42), dim3(256), 0, stream, a);

@@ -24,8 +24,11 @@ __device__ __forceinline__ void wait_vmem() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// 16 bytes per lane from src into LDS at byte offset lds (the wave's base,
-// the same in every lane; lane i writes lds + 16i): global_load_lds_dwordx4.
+// 16 bytes per lane from base + off (base the same in every lane: one scalar
+// pair per operand, where a 64-bit address per lane and operand held the
+// widest shapes at their register limit) into LDS at byte offset lds (the
+// wave's base, the same in every lane; lane i writes lds + 16i):
+// global_load_lds_dwordx4.
 // Written out here because the compiler, lacking alias information, treats
 // every copy still in flight as a write to any LDS address a later ds_read
 // touches, and in some shapes waited for all of them (vmcnt(0)) before each
@@ -34,9 +37,19 @@ __device__ __forceinline__ void wait_vmem() {
 // the barrier) order each copy before the reads of its stage, and the
 // compiler's waits for its own loads stay correct: the copies only make its
 // vmcnt counts more conservative.
-__device__ __forceinline__ void copy_to_lds16(const int8_t* src, uint32_t lds) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(__builtin_amdgcn_readfirstlane(lds))
-                 : "memory");
+__device__ __forceinline__ void copy_to_lds16(const int8_t* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
+}
+
+// Where a wave's copies of weight operand (32-row tile rt, first or second
+// 32-wide block sub of a k step) start, and each lane's offset from there:
+// lane l takes 16 bytes of row l % 32. Tiles past the last are clamped onto
+// it (read, never stored).
+__device__ __forceinline__ const int8_t* weight_operand(const Q8View& w, const int8_t* qs, uint32_t rt, uint32_t sub,
+                                                        uint32_t lane, uint32_t& off) {
+    const uint32_t first = min(2 * rt, w.tiles - 1), r = lane % 32, tile = min(2 * rt + r / 16, w.tiles - 1);
+    off = (tile - first) * w.nb * Q8_TILE_BLOCK_BYTES + (lane / 32) * 256 + (r % 16) * 16;
+    return qs + ((size_t)first * w.nb + sub) * Q8_TILE_BLOCK_BYTES;
 }
 
 // The LDS byte offset of a pointer into LDS: a flat address of LDS is the
