@@ -79,8 +79,8 @@ __global__ __launch_bounds__(64) void attn_q_planes_kernel(const AttnArgs a, uin
         uint32_t out[AP_PLANES][4];
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            int4 v = make_int4(0, 0, 0, 0);
-            if (valid) v = *(const int4*)(q + ds * 64 + dq + 4 * c);
+            int4 v = *(const int4*)(q + ds * 64 + dq + 4 * c);
+            if (!valid) v = make_int4(0, 0, 0, 0);
             const uint64_t d[4] = {digits5(v.x), digits5(v.y), digits5(v.z), digits5(v.w)};
             need = max(need, max(max(limbs_needed(d[0]), limbs_needed(d[1])), max(limbs_needed(d[2]), limbs_needed(d[3]))));
 #pragma unroll
@@ -111,8 +111,12 @@ __global__ __launch_bounds__(256) void attn_kv_planes_kernel(const AttnArgs a, u
     if (tid < 2) s_need[tid] = 1;
     __syncthreads();
 
+    // Every load is unconditional (keys past the last read the last one and
+    // are zeroed after): a load behind a branch is waited for where the
+    // branch joins, so each came in alone (1545 keys: 36 us, 16 now).
     const uint32_t key = ks * 64 + wave * 16 + (lane & 15), dq = (lane >> 4) * 16;
     const bool kvalid = key < nkeys;
+    const int32_t* kc = a.k_cache + (size_t)g * HD * a.k_pos_stride + (kvalid ? key : nkeys - 1);
     const size_t kl = (size_t)a.kv_heads * p.ks_cap * 4 * DS * FRAG;
     int kneed = 1;
 #pragma unroll
@@ -124,7 +128,8 @@ __global__ __launch_bounds__(256) void attn_kv_planes_kernel(const AttnArgs a, u
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const uint32_t dim = ds * 64 + dq + 4 * c + j;
-                v[j] = kvalid ? a.k_cache[((size_t)g * HD + dim) * a.k_pos_stride + key] : 0;
+                v[j] = kc[(size_t)dim * a.k_pos_stride];
+                if (!kvalid) v[j] = 0;
             }
             const uint64_t d[4] = {digits5(v[0]), digits5(v[1]), digits5(v[2]), digits5(v[3])};
             kneed = max(kneed, max(max(limbs_needed(d[0]), limbs_needed(d[1])), max(limbs_needed(d[2]), limbs_needed(d[3]))));
@@ -149,7 +154,8 @@ __global__ __launch_bounds__(256) void attn_kv_planes_kernel(const AttnArgs a, u
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t k = ks * 64 + 16 * t + 4 * gk + i;
-                v[i] = k < nkeys ? a.v_cache[(size_t)k * a.kv_stride + (size_t)g * HD + dim] : 0;
+                v[i] = a.v_cache[(size_t)min(k, nkeys - 1) * a.kv_stride + (size_t)g * HD + dim];
+                if (k >= nkeys) v[i] = 0;
             }
             const uint64_t d[4] = {digits5(v[0]), digits5(v[1]), digits5(v[2]), digits5(v[3])};
             vneed = max(vneed, max(max(limbs_needed(d[0]), limbs_needed(d[1])), max(limbs_needed(d[2]), limbs_needed(d[3]))));
@@ -174,6 +180,24 @@ __global__ __launch_bounds__(256) void attn_kv_planes_kernel(const AttnArgs a, u
 struct PrefillSmem {
     int32_t info[4][16][2];   // per wave and query row: first-maximum key, residual
     int32_t big[4][16][8];    // per wave and query row: large-weight keys (two per lane group, -1 none)
+};
+
+// The d-tiles of one value pass: head size 256 takes four passes of four
+// (two of eight spill), 512 (one wave per SIMD) four of eight.
+constexpr uint32_t value_pass(uint32_t hd) { return hd >= 512 ? 8 : hd >= 256 ? 4 : hd / 16; }
+
+// The waves of a workgroup that share one head's keys meet here: each wave's
+// first maxima and exp sums, the weights' sums, the large weights' keys (at
+// most two per row: w >= BIG_WEIGHT is over 0.498 of the sum), and the value
+// accumulators, added in place.
+constexpr uint32_t KEY_WAVES = 8;
+template <uint32_t HD>
+struct SplitSmem {
+    int32_t best[KEY_WAVES][16];
+    uint32_t best_key[KEY_WAVES][16];
+    double sum[KEY_WAVES][16];
+    int32_t wsum[16], nbig[16], big[16][2];
+    int32_t acc[value_pass(HD)][AP_V_PLANES + 1][4][64];
 };
 
 template <uint32_t HD, int LQK>
@@ -239,9 +263,11 @@ __device__ __forceinline__ void tile_scores(const AttnArgs& a, const v4i (&kf)[L
 }
 
 // One wave: 16 query rows of one head over key steps [ks0, ks1), queries
-// and keys of LQK digits, values of AP_V_PLANES.
-template <uint32_t HD, int LQK>
-__device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens, PrefillSmem& sm, uint32_t g,
+// and keys of LQK digits, values of AP_V_PLANES. SPLIT: the wave's share
+// (possibly none) of the head's key steps, the workgroup's KEY_WAVES waves
+// together covering them.
+template <uint32_t HD, int LQK, bool SPLIT, class Smem>
+__device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens, Smem& sm, uint32_t g,
                                              uint32_t head, uint32_t qt, uint32_t ks0, uint32_t ks1) {
     constexpr uint32_t DS = HD / 64, DT = HD / 16;
     const AttnPlanes& p = a.planes;
@@ -278,7 +304,7 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
     int32_t best = INT32_MIN;
     uint32_t best_key = 0xffffffffu;
     if constexpr (KEY_PREFETCH) {
-        load_key_tile<HD, LQK>(kbase + (size_t)kt0 * DS * FRAG, kl, kf);
+        if (!SPLIT || kt0 < kt1) load_key_tile<HD, LQK>(kbase + (size_t)kt0 * DS * FRAG, kl, kf);
         // Waited for here, where the compiler sees it (s_waitcnt vmcnt(0)):
         // a load into kf still pending at the loop's entry made its wait
         // insertion, which merges the loop's entry with its back edge,
@@ -320,13 +346,34 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
             best_key = ok;
         }
     }
+    if constexpr (SPLIT) {
+        if (lane < 16) {
+            sm.best[wave][lane] = best;
+            sm.best_key[wave][lane] = best_key;
+        }
+        for (uint32_t c = tid; c < sizeof(sm.acc) / 4; c += 64 * KEY_WAVES) (&sm.acc[0][0][0][0])[c] = 0;
+        if (tid < 16) sm.wsum[tid] = 0, sm.nbig[tid] = 0;
+        lds_barrier();
+        best = INT32_MIN;
+        best_key = 0xffffffffu;
+#pragma unroll
+        for (uint32_t v = 0; v < KEY_WAVES; v++) {
+            const int32_t ov = sm.best[v][lane & 15];
+            const uint32_t ok = sm.best_key[v][lane & 15];
+            if (ov > best || (ov == best && ok < best_key)) {
+                best = ov;
+                best_key = ok;
+            }
+        }
+    }
 
     // (2) the sum of exp terms (non-negative, so no order and no saturation)
     // from the stored scores; each lane overwrites a tile's scores with its
     // terms for (3) (2^32, the maximum's term, as 0xffffffff: every other
     // term is below 2^32 - 2^15).
     double fsum = 0;  // at most 2^16 terms of 2^32: exact
-    uint4 sn = *(const uint4*)(estore + (size_t)kt0 * 256);
+    uint4 sn = make_uint4(0, 0, 0, 0);
+    if (!SPLIT || kt0 < kt1) sn = *(const uint4*)(estore + (size_t)kt0 * 256);
     // Waited for here, visibly (as the first key tile above): otherwise
     // each tile's wait for its prefetched scores also covered the previous
     // tile's store of its terms.
@@ -349,6 +396,13 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
     }
     fsum += __shfl_xor(fsum, 16);
     fsum += __shfl_xor(fsum, 32);
+    if constexpr (SPLIT) {
+        if (lane < 16) sm.sum[wave][lane] = fsum;
+        lds_barrier();
+        fsum = 0;
+#pragma unroll
+        for (uint32_t v = 0; v < KEY_WAVES; v++) fsum += sm.sum[v][lane & 15];  // exact in any order
+    }
     const uint64_t sum = (uint64_t)fsum;
     const double q_scale = qvalid ? 4294967296.0 / (double)sum : 0.0;
     const double w_scale = qvalid ? 65536.0 / (double)sum : 0.0;
@@ -368,7 +422,8 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
         const int8_t* vbase = p.v + (size_t)g * p.ks_cap * DT * FRAG + lane * 16;
         int32_t wsum = 0;
         int32_t big[2] = {-1, -1};
-        uint4 en = *(const uint4*)(estore + (size_t)kt0 * 256);
+        uint4 en = make_uint4(0, 0, 0, 0);
+        if (!SPLIT || kt0 < kt1) en = *(const uint4*)(estore + (size_t)kt0 * 256);
 #pragma unroll 1
         for (uint32_t ks = ks0; ks < ks1; ks++) {
             // The step's value operands, needed after its four weight tiles.
@@ -441,6 +496,50 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
         wsum += __shfl_xor(wsum, 16);
         wsum += __shfl_xor(wsum, 32);
 
+        if constexpr (SPLIT) {
+            // The waves' sums meet in LDS; then the workgroup shares the
+            // pass's outputs.
+            if (lane < 16) atomicAdd(&sm.wsum[lane], wsum);
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                if (big[j] >= 0) {
+                    const int slot = atomicAdd(&sm.nbig[lane & 15], 1);
+                    if (slot < 2) sm.big[lane & 15][slot] = big[j];
+                }
+            if (kt0 < kt1) {
+#pragma unroll
+                for (uint32_t dt = 0; dt < DN; dt++)
+#pragma unroll
+                    for (int s = 0; s < AP_V_PLANES + 1; s++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) atomicAdd(&sm.acc[dt][s][i][lane], pacc[dt][s][i]);
+            }
+            // (At the first pass the wave that holds the first maximum's
+            // key; every wave computed the same one.)
+            if (wave == 0 && lane < 16) sm.best_key[0][lane] = best_key;
+            lds_barrier();
+            const int32_t* vcache = a.v_cache + (size_t)g * HD;
+            for (uint32_t c = tid; c < DN * 256; c += 64 * KEY_WAVES) {
+                const uint32_t l = c % 64, i = c / 64 % 4, dt = c / 256, qq = 4 * (l / 16) + i, row = qt * 16 + qq;
+                if (row >= tokens) continue;
+                const uint32_t dim = (D0 + dt) * 16 + l % 16;
+                uint64_t tot = 0;
+#pragma unroll
+                for (int s = 0; s < AP_V_PLANES + 1; s++) tot += (uint64_t)(int64_t)sm.acc[dt][s][i][l] << (8 * s);
+                const int64_t resid = dn::sub_sat(dn::ONE_ACT, sm.wsum[qq]);
+                tot += (uint64_t)(resid * vcache[(size_t)sm.best_key[0][qq] * a.kv_stride + dim]);
+                for (int j = 0; j < sm.nbig[qq]; j++)
+                    tot += (uint64_t)((int64_t)65536 * vcache[(size_t)sm.big[qq][j] * a.kv_stride + dim]);
+                a.ctx[(size_t)row * a.ctx_stride + (size_t)head * HD + dim] = dn::requantize((int64_t)tot);
+            }
+            if constexpr (D0 + DN < DT) {  // another pass
+                lds_barrier();
+                for (uint32_t c = tid; c < sizeof(sm.acc) / 4; c += 64 * KEY_WAVES) (&sm.acc[0][0][0][0])[c] = 0;
+                if (tid < 16) sm.wsum[tid] = 0, sm.nbig[tid] = 0;
+                lds_barrier();
+            }
+            return;
+        } else {
         // Per query row: the residual goes to the first maximum; every large
         // weight adds 65536 * v back. (Each wave reads only its own rows'
         // entries; a second pass rewrites them with the same values.)
@@ -476,10 +575,9 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
                 a.ctx[(size_t)row * a.ctx_stride + (size_t)head * HD + dim] = dn::requantize((int64_t)tot);
             }
         }
+        }
     };
-    // Head size 256: four passes of four d-tiles (two of eight spill);
-    // 512 (one wave per SIMD): four passes of eight.
-    constexpr uint32_t VPASS = HD >= 512 ? 8 : HD >= 256 ? 4 : DT;
+    constexpr uint32_t VPASS = value_pass(HD);
     auto passes = [&](auto self, auto pc) __attribute__((always_inline)) {
         constexpr uint32_t P = decltype(pc)::value;
         values_pass(std::integral_constant<uint32_t, P * VPASS>{}, std::integral_constant<uint32_t, VPASS>{});
@@ -527,10 +625,60 @@ __global__ __launch_bounds__(256, HD >= 512 ? 1 : 2) void attn_prefill_kernel(co
     if (limbs > AP_PLANES) {
         for (uint32_t i = 0; i < 4 * rows; i++) attend_row(a, h0 + i / rows, qt * 16 + i % rows, sm.row);
     } else if (limbs <= 3) {
-        prefill_wave<HD, 3>(a, tokens, sm.pre, (h0 + wave) / group, h0 + wave, qt, ks0, ks1);
+        prefill_wave<HD, 3, false>(a, tokens, sm.pre, (h0 + wave) / group, h0 + wave, qt, ks0, ks1);
     } else {
-        prefill_wave<HD, 4>(a, tokens, sm.pre, (h0 + wave) / group, h0 + wave, qt, ks0, ks1);
+        prefill_wave<HD, 4, false>(a, tokens, sm.pre, (h0 + wave) / group, h0 + wave, qt, ks0, ks1);
     }
+}
+
+// Launches of few query tiles: one head over one 16-row query tile per
+// workgroup, its key steps dealt to eight waves in consecutive runs, so that
+// the three serial walks over the keys are an eighth as long.
+template <uint32_t HD>
+__global__ __launch_bounds__(64 * KEY_WAVES, 2) void attn_prefill_split_kernel(const AttnArgs a, uint32_t tokens) {
+    __shared__ union {
+        AttnRowSmem row;
+        SplitSmem<HD> split;
+    } sm;
+    __shared__ int s_limbs;
+    const AttnPlanes& p = a.planes;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    const uint32_t QT = (tokens + 15) / 16;
+    const uint32_t qt = QT - 1 - blockIdx.x / a.heads, head = blockIdx.x % a.heads, g = head / (a.heads / a.kv_heads);
+    const uint32_t pos0 = (uint32_t)(*a.d_pos);
+    const uint32_t rows = min(16u, tokens - qt * 16);
+    const uint32_t first_pos = pos0 + qt * 16, last_pos = first_pos + rows - 1;
+    const uint32_t first_key = (a.window == 0 || first_pos + 1 <= a.window) ? 0 : first_pos + 1 - a.window;
+    const uint32_t ks0 = first_key / 64, n = last_pos / 64 + 1 - ks0;
+
+    // Digits the block's queries and keys need, as in attn_prefill_kernel.
+    if (tid == 0) s_limbs = (int)p.q_limbs[head * p.qt_cap + qt];
+    __syncthreads();
+    const uint8_t* kvl = p.kv_limbs + (size_t)g * p.ks_cap * 2;
+    for (uint32_t ks = ks0 + tid; ks < ks0 + n; ks += 64 * KEY_WAVES)
+        atomicMax(&s_limbs, kvl[2 * ks + 1] > AP_V_PLANES ? AP_PLANES + 1 : (int)kvl[2 * ks]);
+    __syncthreads();
+    const int limbs = s_limbs;
+    const uint32_t mine0 = ks0 + n * wave / KEY_WAVES, mine1 = ks0 + n * (wave + 1) / KEY_WAVES;
+    if (limbs > AP_PLANES) {
+        for (uint32_t i = 0; i < rows; i++) attend_row(a, head, qt * 16 + i, sm.row);
+    } else if (limbs <= 3) {
+        prefill_wave<HD, 3, true>(a, tokens, sm.split, g, head, qt, mine0, mine1);
+    } else {
+        prefill_wave<HD, 4, true>(a, tokens, sm.split, g, head, qt, mine0, mine1);
+    }
+}
+
+// Whether a launch's keys are split over the waves: while the four-head
+// workgroups leave no CU two of them. us per layer at head size 128, 32
+// heads, four heads per workgroup / split:
+//   2 rows after 1500 keys  180 / 42    45 after 1500  175 / 42   100 after 700  100 / 32
+//   200 after 1500          186 / 93   512 after 512   124 / 116  200 after 0     41 / 33
+//   700 after 0              88 / 112  1024 after 1000 322 / 358  2048 after 0   435 / 540
+// Head size 256 only below the bound of iris_attention_prefill_applies.
+bool prefill_split(const AttnArgs& a, uint32_t tokens) {
+    const uint32_t wgs = (tokens + 15) / 16 * (a.heads / 4);
+    return a.head_dim <= 128 ? wgs <= (uint32_t)iris_device_cus() : a.head_dim == 256 && wgs < 128;
 }
 
 template <uint32_t HD>
@@ -539,6 +687,12 @@ int prefill_launch(const AttnArgs& a, uint32_t tokens, hipStream_t stream) {
     hipLaunchKernelGGL(attn_q_planes_kernel<HD>, dim3(QT, a.heads), dim3(64), 0, stream, a, tokens);
     hipLaunchKernelGGL(attn_kv_planes_kernel<HD>, dim3(a.planes.ks_cap, a.kv_heads), dim3(256), 0, stream, a, tokens);
     const uint32_t wgs = QT * (a.heads / 4);
+    if constexpr (HD <= 256) {
+        if (prefill_split(a, tokens)) {
+            hipLaunchKernelGGL(attn_prefill_split_kernel<HD>, dim3(QT * a.heads), dim3(64 * KEY_WAVES), 0, stream, a, tokens);
+            return (int)hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL(attn_prefill_kernel<HD>, dim3(wgs), dim3(256), 0, stream, a, tokens);
     return (int)hipGetLastError();
 }
@@ -573,7 +727,11 @@ bool iris_attention_prefill_applies(const AttnArgs& a, uint32_t tokens, uint32_t
     // 12.8 ms for 128 rows on the one-row routine), and so does 512 (one
     // wave per SIMD; the scaled gemma-4 shape: 12.5 against 16.7 ms for 2048
     // rows, 5.2 against 4.9 ms for 600).
-    if (a.head_dim >= 256 && (tokens + 15) / 16 * (a.heads / 4) < 128) return false;
+    // Head size 256 with its keys split over the waves from 192 workgroups of
+    // one head (three Gemma-2B-shape layers: 300 rows 3.55 ms either way, 512
+    // rows 4.90 against 5.22 ms, 128 rows 1.93 against 1.80).
+    const uint32_t tiles = (tokens + 15) / 16;
+    if (a.head_dim >= 256 && tiles * (a.heads / 4) < 128 && !(a.head_dim == 256 && tiles * a.heads >= 192)) return false;
     return tokens >= 2 && p.q && p.k && p.v && p.q_limbs && p.kv_limbs && p.e_store &&
            (a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256 || a.head_dim == 512) &&
            a.heads % a.kv_heads == 0 && a.heads % 4 == 0 && (tokens + 15) / 16 <= p.qt_cap &&

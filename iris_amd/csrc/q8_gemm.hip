@@ -85,8 +85,8 @@ __global__ __launch_bounds__(256) void digit_planes_kernel(const GemvArgs a) {
         uint32_t out[PL_MAX][4];
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            int4 v = make_int4(0, 0, 0, 0);
-            if (valid) v = *(const int4*)(x + k0 + 4 * c);
+            int4 v = *(const int4*)(x + k0 + 4 * c);  // not behind a branch: all are in flight together
+            if (!valid) v = make_int4(0, 0, 0, 0);
             if (norm) {
                 const int4 nw = *(const int4*)(a.norm_w + k0 + 4 * c);
                 v.x = dn::mul_sat(dn::mul_sat(v.x, scale), nw.x);
