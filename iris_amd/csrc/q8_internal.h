@@ -22,6 +22,7 @@ enum Q8ScaleMode : int {
     Q8_SCALE_ROW = 0,  // every block of a row shares one scale: one i64 Q.24 per row
     Q8_SCALE_F16 = 1,  // one f16 per block (the reference's encoding)
     Q8_SCALE_I64 = 2,  // one arbitrary i64 Q.24 per block (q8gpu_upload's input)
+    Q16_PLANES = 3,    // no Q8_0 blocks: a Q16.16 matrix as two digit planes (Q16Planes)
 };
 
 // Rows per tile and the tiled byte layout:
@@ -66,6 +67,20 @@ struct Q8GpuMatrix {
     bool fold_tried;  // the folding was attempted (prepared or refused)
 };
 
+// A Q16.16 matrix whose values need at most two signed byte digits
+// (|w| < 2^15), as two digit planes in the qs tile layout, for multi-token
+// products on the matrix cores. Such a product is sum_k w_k x_k, |.| < 2^60
+// for cols <= 16384, rounded at 16 fraction bits (dot_bits, tensor.rs:522-528,
+// then requantize, ops.rs:448-451): a folded row of shift 8 rounded at 24.
+struct Q16Planes {
+    int8_t* planes = nullptr;  // null: not built (wider values, or a width the tiles do not take)
+    int32_t* shift = nullptr;  // [tiles * 16], 8
+    bool tried = false;
+};
+// Builds p from w [rows][cols] in device memory (once; 2 bytes per value).
+int iris_q16_prepare(const int32_t* w, uint32_t rows, uint32_t cols, Q16Planes* p, hipStream_t stream);
+void iris_q16_free(Q16Planes* p);
+
 // Kernel-side view of a matrix.
 struct Q8View {
     const uint8_t* qs;
@@ -84,6 +99,14 @@ inline Q8View q8_view(const Q8GpuMatrix* m) {
     return Q8View{m->qs,   m->sc16,       m->sc64,       m->row_scale,      m->rows,        m->cols,
                   m->nb,   m->tiles,      m->scale_mode, m->fold.planes,    m->fold.shift,  m->fold.nplanes,
                   m->digits_bound};
+}
+
+inline Q8View q16_view(const Q16Planes& p, uint32_t rows, uint32_t cols) {
+    Q8View v{};
+    v.rows = rows, v.cols = cols, v.nb = cols / 32, v.tiles = (rows + Q8_TILE_ROWS - 1) / Q8_TILE_ROWS;
+    v.scale_mode = Q16_PLANES;
+    v.fold_planes = p.planes, v.fold_shift = p.shift, v.fold_nplanes = 2;
+    return v;
 }
 
 // Builds m's folded planes (once; per-block scale matrices only) so that
@@ -115,6 +138,7 @@ enum GemvEpilogue : int {
                        // (mistral consecutive pairs), q -> out, k/v -> caches
     EPI_HEAD_SELECT = 6,  // logits = softcap(value) and each tile's first maximum
                           // to sel_partial, for iris_select_launch
+    EPI_GELU_MUL = 7,  // Q16_PLANES products: out = mul_sat(gelu(value), residual)
 };
 
 struct GemvArgs {

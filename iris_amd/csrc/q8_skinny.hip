@@ -21,6 +21,9 @@
 // tokens 81 -> 22; and where an unfolded per-block matrix went through the
 // one-token kernel once per token, 24 tokens of 4096 x 4096 93 -> 22.
 //
+// Q16.16 matrices (the per-layer-embedding projections of gemma-dense) come
+// as two digit planes made once, a step of both read as they are.
+//
 // Two shapes: SH = 16 (16 rows x 16 tokens, v_mfma_i32_16x16x64_i8, twice
 // the workgroups) for up to 16 tokens, SH = 32 (32 x 32,
 // v_mfma_i32_32x32x32_i8) for more, one 32-token tile per workgroup; the
@@ -86,7 +89,8 @@ template <int SH, int MODE, int LG, int DEPTH, uint32_t SK_WAVES>
 __device__ __forceinline__ void skinny_tile(const GemvArgs& a, int32_t* smem, uint32_t rt, uint32_t tt) {
     using S = Shape<SH>;
     using Acc = typename S::Acc;
-    constexpr int WP = MODE == Q8_SCALE_ROW ? 1 : 3, NS = WP + LG - 1;
+    constexpr int WP = MODE == Q8_SCALE_ROW ? 1 : MODE == Q16_PLANES ? 2 : 3, NS = WP + LG - 1;
+    constexpr int QP = MODE == Q16_PLANES ? 2 : 1;  // weight planes read
     constexpr uint32_t SK_THREADS = 64 * SK_WAVES;
     const Q8View& w = a.w;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -95,8 +99,9 @@ __device__ __forceinline__ void skinny_tile(const GemvArgs& a, int32_t* smem, ui
     // This lane's row, its 16 bytes of a step's weights and its scale.
     const uint32_t r = lane % SH, tile16 = SH == 16 ? rt : min(2 * rt + r / 16, w.tiles - 1);
     const uint32_t row = tile16 * 16 + r % 16;
-    const uint8_t* qp = w.qs + (size_t)tile16 * KB * Q8_TILE_BLOCK_BYTES +
+    const uint8_t* qp = (MODE == Q16_PLANES ? (const uint8_t*)w.fold_planes : w.qs) + (size_t)tile16 * KB * Q8_TILE_BLOCK_BYTES +
                         (SH == 16 ? lane * 16 : (lane / 32) * 256 + (r % 16) * 16);
+    const size_t qstride = (size_t)w.tiles * KB * Q8_TILE_BLOCK_BYTES;
     const uint16_t* sp = MODE == Q8_SCALE_F16 ? w.sc16 + ((size_t)tile16 * KB + (SH == 16 ? lane / 32 : 0)) * 16 + r % 16
                                               : nullptr;
     const int32_t least = MODE == Q8_SCALE_F16 ? w.fold_shift[row] : 0;
@@ -108,21 +113,24 @@ __device__ __forceinline__ void skinny_tile(const GemvArgs& a, int32_t* smem, ui
     Acc acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) acc[s] = Acc{};
-    v4i q[DEPTH], b[DEPTH][LG];
+    v4i q[DEPTH][QP], b[DEPTH][LG];
     uint32_t sc[DEPTH];
     auto load = [&](int u, uint32_t step) __attribute__((always_inline)) {
         // Past the end: the last step again (never used), so no branch
         // separates the loads from their waits.
         const uint32_t kb = min(step, steps - 1) * S::NB;
-        q[u] = *(const v4i*)(qp + (size_t)kb * Q8_TILE_BLOCK_BYTES);
+#pragma unroll
+        for (int p = 0; p < QP; p++) q[u][p] = *(const v4i*)(qp + p * qstride + (size_t)kb * Q8_TILE_BLOCK_BYTES);
         if (MODE == Q8_SCALE_F16) sc[u] = sp[(size_t)kb * 16];
 #pragma unroll
         for (int l = 0; l < LG; l++) b[u][l] = *(const v4i*)(bp + l * lstride + (size_t)kb * FRAG);
     };
     auto compute = [&](int u) __attribute__((always_inline)) {
-        if (MODE == Q8_SCALE_ROW) {
+        if (MODE != Q8_SCALE_F16) {
 #pragma unroll
-            for (int l = 0; l < LG; l++) acc[l] = S::mfma(q[u], b[u][l], acc[l]);
+            for (int l = 0; l < LG; l++)
+#pragma unroll
+                for (int p = 0; p < QP; p++) acc[p + l] = S::mfma(q[u][p], b[u][l], acc[p + l]);
         } else {
             const uint32_t e = (sc[u] >> 10) & 0x1f, mant = sc[u] & 0x3ff;
             const int32_t m = (int32_t)(e ? 1024 + mant : mant);
@@ -131,7 +139,7 @@ __device__ __forceinline__ void skinny_tile(const GemvArgs& a, int32_t* smem, ui
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 int d[3];
-                weight_digits((uint32_t)q[u][c], f, d, 0x808080);
+                weight_digits((uint32_t)q[u][0][c], f, d, 0x808080);
 #pragma unroll
                 for (int p = 0; p < WP; p++) wd[p][c] = d[p];
             }
@@ -202,7 +210,11 @@ __device__ __forceinline__ void skinny_tile(const GemvArgs& a, int32_t* smem, ui
     if (a.epilogue != EPI_SWIGLU && a.epilogue != EPI_GEGLU) {
         for (uint32_t c = tid; c < SH * SH; c += SK_THREADS) {
             const uint32_t rl = c % SH, tl = c / SH;
-            if (row0 + rl < w.rows && tok0 + tl < a.tokens)
+            if (row0 + rl >= w.rows || tok0 + tl >= a.tokens) continue;
+            if (MODE == Q16_PLANES && a.epilogue == EPI_GELU_MUL)
+                a.out[(size_t)(tok0 + tl) * a.out_stride + row0 + rl] = dn::mul_sat(
+                    dn::gelu(smem[rl * STRIDE + tl]), a.residual[(size_t)(tok0 + tl) * a.residual_stride + row0 + rl]);
+            else
                 store_output(a, row0 + rl, tok0 + tl, smem[rl * STRIDE + tl], smem[(rl ^ 1) * STRIDE + tl]);
         }
         return;
@@ -294,6 +306,9 @@ bool iris_skinny_applies(const GemvArgs& a) {
         a.prologue == PRO_NORM_RES_NORM || a.tokens > 65535)
         return false;
     if (a.w.scale_mode == Q8_SCALE_ROW) return a.w.cols < (1u << 17) && few_tiles(a);
+    // The planes' only path, whatever the tokens (two shared-shift terms).
+    if (a.w.scale_mode == Q16_PLANES)
+        return a.w.cols <= 16384 && (a.epilogue == EPI_STORE || a.epilogue == EPI_GELU_MUL);
     // Per-block scales: three weight digits suffice (the upload's bound) and
     // the shared-shift sums stay below 2^31. Without folded planes this is
     // the only matrix-core path, whatever the tokens; work space that is not
@@ -312,6 +327,8 @@ int iris_skinny_launch(const GemvArgs& a, hipStream_t stream) {
         constexpr uint32_t W = decltype(w)::value;
         if (a.w.scale_mode == Q8_SCALE_ROW)
             hipLaunchKernelGGL((q8_skinny_kernel<SH, Q8_SCALE_ROW, W>), grid, dim3(64 * W), 0, stream, a, row_tiles, tok_tiles);
+        else if (a.w.scale_mode == Q16_PLANES)
+            hipLaunchKernelGGL((q8_skinny_kernel<SH, Q16_PLANES, W>), grid, dim3(64 * W), 0, stream, a, row_tiles, tok_tiles);
         else
             hipLaunchKernelGGL((q8_skinny_kernel<SH, Q8_SCALE_F16, W>), grid, dim3(64 * W), 0, stream, a, row_tiles, tok_tiles);
     };

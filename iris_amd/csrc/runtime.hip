@@ -405,6 +405,11 @@ void iris_model_free(IrisModel* m) {
                            L.k_norm, L.ple_gate, L.ple_proj})
             hipFree(p);
     }
+    for (auto& L : m->layers) {
+        iris_q16_free(&L.ple_gate_planes);
+        iris_q16_free(&L.ple_proj_planes);
+    }
+    iris_q16_free(&m->ple_model_planes);
     q8gpu_free(m->head);
     hipFree(m->embed_raw);
     hipFree(m->final_norm);
@@ -610,6 +615,30 @@ static int mistral_pass(IrisSession* s, uint32_t rows, const CkptSink* sink) {
 //
 // The PLE inputs of every layer (view_kernels.rs:59-99) from the embedded
 // rows in s->x and their ids, into s->ple_rows [rows][layers * ple_width].
+// A Q16.16 product of a pass: on the matrix cores where its planes were
+// built and the rows are enough, else one row at a time. us of a prompt pass
+// of three Gemma-2B-shape layers (seven such products), row by row / planes:
+// 512 rows 4822 / 2744, 128 rows 1736 / 1251, 64 rows 1301 / 1087, 32 rows
+// 1102 / 1041, 16 rows 878 / 873, 8 rows 834 / 875.
+constexpr uint32_t Q16_PLANES_MIN_ROWS = 24;
+static int i32_product(IrisSession* s, const I32GemvArgs& ig, const Q16Planes& planes, uint32_t rows) {
+    if (rows < Q16_PLANES_MIN_ROWS || !planes.planes || ig.res_in || ig.ssq_out)
+        return iris_i32_gemv_launch(ig, rows, s->stream);
+    GemvArgs g{};
+    g.w = q16_view(planes, ig.rows, ig.cols);
+    g.x = ig.x;
+    g.x_stride = ig.x_stride;
+    g.tokens = rows;
+    g.prologue = PRO_NONE;
+    g.epilogue = ig.aux ? EPI_GELU_MUL : EPI_STORE;
+    g.out = ig.out;
+    g.out_stride = ig.out_stride;
+    g.residual = ig.aux;
+    g.residual_stride = ig.aux_stride;
+    with_gemm_space(g, s, rows);
+    return iris_gemm_launch(g, s->stream);
+}
+
 static int gemma_ple(IrisSession* s, uint32_t rows) {
     IrisModel* m = s->model;
     const IrisModelDesc& d = m->d;
@@ -623,7 +652,7 @@ static int gemma_ple(IrisSession* s, uint32_t rows) {
     ig.x_stride = H;
     ig.out = s->ple_proj;
     ig.out_stride = LP;
-    RT_CHECK(iris_i32_gemv_launch(ig, rows, st));
+    RT_CHECK(i32_product(s, ig, m->ple_model_planes, rows));
     PleArgs pa{};
     pa.proj = s->ple_proj;
     pa.row_stride = LP;
@@ -828,7 +857,7 @@ static int gemma_layer(IrisSession* s, uint32_t l, uint32_t rows, bool carry) {
             ig.ssq_n = h_tiles;
             ig.res_out = xin;
         }
-        RT_CHECK(iris_i32_gemv_launch(ig, rows, st));
+        RT_CHECK(i32_product(s, ig, L.ple_gate_planes, rows));
         ig = I32GemvArgs{};
         ig.w = L.ple_proj;
         ig.rows = H;
@@ -838,7 +867,7 @@ static int gemma_layer(IrisSession* s, uint32_t l, uint32_t rows, bool carry) {
         ig.out = s->tmp;
         ig.out_stride = H;
         if (carry) ig.ssq_out = s->ssq_x;
-        RT_CHECK(iris_i32_gemv_launch(ig, rows, st));
+        RT_CHECK(i32_product(s, ig, L.ple_proj_planes, rows));
         if (carry) {
             c.pending = true;
             c.norm_w = L.norm_post_ple;
@@ -1132,9 +1161,18 @@ int iris_session_create(IrisModel* m, uint32_t max_positions, uint32_t max_rows,
         for (uint32_t l = 0; l < d.layers && st == hipSuccess; l++)
             for (Q8GpuMatrix* w : {m->layers[l].wqkv, m->layers[l].wo, m->layers[l].wgu, m->layers[l].wdown})
                 if (st == hipSuccess) st = (hipError_t)iris_q8_prepare_fold(w, s->stream);
+        // So do gemma-dense's Q16.16 projections, as digit planes.
+        if (d.family == IRIS_FAMILY_GEMMA_DENSE) {
+            const uint32_t lp = d.layers * d.ple_width;
+            if (st == hipSuccess) st = (hipError_t)iris_q16_prepare(m->ple_model_proj, lp, d.hidden, &m->ple_model_planes, s->stream);
+            for (auto& L : m->layers) {
+                if (st == hipSuccess) st = (hipError_t)iris_q16_prepare(L.ple_gate, d.ple_width, d.hidden, &L.ple_gate_planes, s->stream);
+                if (st == hipSuccess) st = (hipError_t)iris_q16_prepare(L.ple_proj, d.hidden, d.ple_width, &L.ple_proj_planes, s->stream);
+            }
+        }
         // The matrix-core SwiGLU epilogues look silu up.
         if (d.family != IRIS_FAMILY_GEMMA_DENSE && st == hipSuccess) st = (hipError_t)iris_silu_table(&s->silu_tab);
-        size_t widest = std::max<size_t>(d.hidden, std::max<size_t>(qw, m->max_ffn));
+        size_t widest = std::max<size_t>({d.hidden, qw, m->max_ffn, d.family == IRIS_FAMILY_GEMMA_DENSE ? d.ple_width : 0});
         if (st == hipSuccess) st = hipMalloc((void**)&s->planes, gemm_planes_bytes((uint32_t)widest, max_rows));
         alloc(&s->token_limbs, (size_t)gemm_limb_ints((uint32_t)widest, max_rows));
         if (st == hipSuccess) st = hipMalloc((void**)&s->gated_gemm_planes, gemm_planes_bytes(m->max_ffn, max_rows));

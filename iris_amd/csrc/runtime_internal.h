@@ -29,6 +29,7 @@ struct LayerWeights {
     int32_t* k_norm = nullptr;
     int32_t* ple_gate = nullptr;       // per_layer_input_gate, Q16.16 [ple][hidden]
     int32_t* ple_proj = nullptr;       // per_layer_projection, Q16.16 [hidden][ple]
+    Q16Planes ple_gate_planes, ple_proj_planes;  // of the two, for multi-row passes
     int32_t layer_scalar = 0;          // 0 = absent
     // derived at finalize (model.rs:817-877)
     uint32_t head_dim = 0, rotary_dim = 0, window = 0;
@@ -57,6 +58,7 @@ struct IrisModel {
     uint8_t* embed_ple = nullptr;        // embed_tokens_per_layer, reference Q8_0 rows
     uint32_t embed_ple_row_bytes = 0;
     int32_t* ple_model_proj = nullptr;   // per_layer_model_projection, Q16.16 [layers*ple][hidden]
+    Q16Planes ple_model_planes;          // its planes, for multi-row passes
     int32_t* ple_proj_norm = nullptr;    // per_layer_projection_norm [ple]
     int64_t* rope_sliding = nullptr;     // frequency ladders of the two layer kinds
     int64_t* rope_full = nullptr;
