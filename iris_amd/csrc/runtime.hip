@@ -1241,6 +1241,10 @@ void iris_session_free(IrisSession* s) {
     hipFree(s->attn_planes.e_store);
     hipFree(s->rope_sc);
     hipFree(s->kv_stage);
+    if (s->copy_stream) (void)hipStreamSynchronize(s->copy_stream);
+    if (s->logits_ring) (void)hipHostFree(s->logits_ring);
+    for (auto e : s->logits_events)
+        if (e) (void)hipEventDestroy(e);
     hipFree(s->ckpt_dev);
     if (s->ckpt_host) hipHostFree(s->ckpt_host);
     for (auto e : s->ckpt_events)
@@ -1248,6 +1252,21 @@ void iris_session_free(IrisSession* s) {
     if (s->copy_stream) hipStreamDestroy(s->copy_stream);
     if (s->stream) hipStreamDestroy(s->stream);
     delete s;
+}
+
+constexpr size_t LOGITS_RUN = (size_t)1 << 20;  // bytes of kept logits that go to the host together, about
+
+static int ensure_logits_ring(IrisSession* s, size_t slot) {
+    if (!s->copy_stream) RT_CHECK(hipStreamCreate(&s->copy_stream));
+    for (auto& e : s->logits_events)
+        if (!e) RT_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (slot <= s->logits_slot) return 0;
+    if (s->logits_ring) RT_CHECK(hipHostFree(s->logits_ring));
+    s->logits_ring = nullptr;
+    s->logits_slot = 0;
+    RT_CHECK(hipHostMalloc((void**)&s->logits_ring, LOGITS_SLOTS * slot, hipHostMallocDefault));
+    s->logits_slot = slot;
+    return 0;
 }
 
 static int session_generate(IrisSession* s, const int32_t* prompt, uint32_t prompt_len, uint32_t tokens,
@@ -1277,15 +1296,44 @@ static int session_generate(IrisSession* s, const int32_t* prompt, uint32_t prom
     // The passes fill positions 0..prompt_len + tokens - 1 of every cache
     // (covered once they have run).
     uncover_all(s, 0, (uint32_t)end, true);
+    // Kept logits leave for the host some steps at a time while the next
+    // steps run: into a pinned slot on the copy stream, from there to the
+    // caller's rows, LOGITS_SLOTS runs of steps behind at most.
+    const size_t row = (size_t)d.vocab * 4;
+    const uint32_t run = (uint32_t)std::max<size_t>(1, LOGITS_RUN / row);
+    if (out_logits) RT_CHECK(ensure_logits_ring(s, std::min(run, tokens) * row));
+    uint32_t sent = 0, runs = 0, drained = 0;  // steps, runs
+    auto drain = [&]() -> int {
+        const uint32_t slot = drained % LOGITS_SLOTS, from = drained * run, n = std::min(run, tokens - from);
+        RT_CHECK(hipEventSynchronize(s->logits_events[LOGITS_SLOTS + slot]));
+        std::memcpy((uint8_t*)out_logits + from * row, s->logits_ring + slot * s->logits_slot, n * row);
+        drained++;
+        return 0;
+    };
+    auto step_done = [&](uint32_t t) -> int {  // step t's launches are in the stream
+        if (!out_logits || (t + 1 - sent < run && t + 1 < tokens)) return 0;
+        if (runs - drained == LOGITS_SLOTS) RT_CHECK(drain());
+        const uint32_t slot = runs % LOGITS_SLOTS;
+        RT_CHECK(hipEventRecord(s->logits_events[slot], s->stream));
+        RT_CHECK(hipStreamWaitEvent(s->copy_stream, s->logits_events[slot], 0));
+        RT_CHECK(hipMemcpyAsync(s->logits_ring + slot * s->logits_slot, (const uint8_t*)s->logits_keep + sent * row,
+                                (t + 1 - sent) * row, hipMemcpyDeviceToHost, s->copy_stream));
+        RT_CHECK(hipEventRecord(s->logits_events[LOGITS_SLOTS + slot], s->copy_stream));
+        sent = t + 1;
+        runs++;
+        return 0;
+    };
     RT_CHECK(session_reset_and_embed(s, prompt, prompt_len));
     RT_CHECK(session_pass(s, prompt_len, nullptr));
     RT_CHECK(session_head_select(s, prompt_len));
     if (use_graph && tokens > 1) RT_CHECK(ensure_graph(s, true));
-    for (uint32_t t = 1; t < tokens; t++) RT_CHECK(session_decode_pass(s, use_graph));
+    RT_CHECK(step_done(0));
+    for (uint32_t t = 1; t < tokens; t++) {
+        RT_CHECK(session_decode_pass(s, use_graph));
+        RT_CHECK(step_done(t));
+    }
+    while (drained < runs) RT_CHECK(drain());
     RT_CHECK(hipMemcpyAsync(out_tokens, s->tokens, (size_t)tokens * 4, hipMemcpyDeviceToHost, s->stream));
-    if (out_logits)
-        RT_CHECK(hipMemcpyAsync(out_logits, s->logits_keep, (size_t)tokens * d.vocab * 4, hipMemcpyDeviceToHost,
-                                s->stream));
     RT_CHECK(hipStreamSynchronize(s->stream));
     // Stop at the first EOS (it is kept), as executor.rs:163-168 does; the
     // passes after it do not change the tokens before it.
@@ -1310,8 +1358,10 @@ static int session_generate(IrisSession* s, const int32_t* prompt, uint32_t prom
 extern "C" int iris_session_generate(IrisSession* s, const int32_t* prompt, uint32_t prompt_len, uint32_t tokens,
                                      const int32_t* eos_ids, uint32_t n_eos, int32_t* out_tokens,
                                      uint32_t* out_count, int32_t* out_logits, int32_t use_graph) {
-    return session_generate(s, prompt, prompt_len, tokens, eos_ids, n_eos, out_tokens, out_count, out_logits,
-                            use_graph);
+    const int st = session_generate(s, prompt, prompt_len, tokens, eos_ids, n_eos, out_tokens, out_count, out_logits,
+                                    use_graph);
+    if (st && s && s->copy_stream) (void)hipStreamSynchronize(s->copy_stream);  // copies a failed run left under way
+    return st;
 }
 
 // Staging for the per-layer checkpoints of passes of up to max_rows rows:
@@ -1322,8 +1372,8 @@ static int ensure_checkpoint_space(IrisSession* s) {
     const size_t bytes = (size_t)d.layers * s->max_rows * d.hidden * 4;
     RT_CHECK(hipMalloc((void**)&s->ckpt_dev, bytes));
     RT_CHECK(hipHostMalloc((void**)&s->ckpt_host, bytes, hipHostMallocDefault));
-    RT_CHECK(hipStreamCreate(&s->copy_stream));
-    s->ckpt_events.assign(2 * (size_t)d.layers, nullptr);
+    if (!s->copy_stream) RT_CHECK(hipStreamCreate(&s->copy_stream));
+    s->ckpt_events.assign((1 + CKPT_PIECES) * (size_t)d.layers, nullptr);
     for (auto& e : s->ckpt_events) RT_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return 0;
 }
@@ -1367,27 +1417,45 @@ static int layer_range_run(IrisSession* s, const int32_t* ids, uint32_t count, u
     const CkptSink sink{s->ckpt_dev, on_device};
     RT_CHECK(session_reset_and_embed(s, ids, count, start_position));
     RT_CHECK(session_pass(s, count, &sink));
+    // A layer's hash is one serial chain over its rows (about 2 GB/s), the
+    // longest part of a pass of few layers, so it starts with the first
+    // quarter to arrive and nothing else runs in its thread: the copies into
+    // the caller's rows, with their page faults, are other jobs.
+    const size_t bytes = n * 4, piece = (bytes / CKPT_PIECES + 4095) / 4096 * 4096;
+    auto piece_of = [&](uint32_t i) { return std::min(bytes, i * piece); };
     for (uint32_t l = 0; l < layers; l++) {
         RT_CHECK(hipStreamWaitEvent(s->copy_stream, on_device[l], 0));
-        RT_CHECK(hipMemcpyAsync(s->ckpt_host + l * n * 4, s->ckpt_dev + l * n, n * 4, hipMemcpyDeviceToHost,
-                                s->copy_stream));
-        RT_CHECK(hipEventRecord(on_host[l], s->copy_stream));
+        for (uint32_t i = 0; i < CKPT_PIECES; i++) {
+            const size_t from = piece_of(i), to = piece_of(i + 1);
+            if (to > from)
+                RT_CHECK(hipMemcpyAsync(s->ckpt_host + l * bytes + from, (const uint8_t*)(s->ckpt_dev + l * n) + from,
+                                        to - from, hipMemcpyDeviceToHost, s->copy_stream));
+            RT_CHECK(hipEventRecord(on_host[l * CKPT_PIECES + i], s->copy_stream));
+        }
     }
     const unsigned hw = std::thread::hardware_concurrency();
-    const uint32_t workers = std::max(1u, std::min({layers, 16u, hw ? hw : 1u}));
+    const uint32_t jobs = 2 * layers;  // even: a layer's hash, odd: its rows
+    const uint32_t workers = std::max(1u, std::min({jobs, 16u, hw ? hw : 1u}));
     std::atomic<int> status{0};
     std::vector<std::thread> pool;
     for (uint32_t t = 0; t < workers; t++)
         pool.emplace_back([&, t] {
-            for (uint32_t l = t; l < layers; l += workers) {
-                const hipError_t st = hipEventSynchronize(on_host[l]);
-                if (st != hipSuccess) {
-                    status = (int)st;
-                    continue;
+            for (uint32_t job = t; job < jobs; job += workers) {
+                const uint32_t l = job / 2;
+                const bool hash = job % 2 == 0;
+                if (hash ? !out_hashes : !out_rows) continue;
+                const uint8_t* rows = s->ckpt_host + l * bytes;
+                Sha256 sha;
+                hipError_t st = hipSuccess;
+                for (uint32_t i = 0; i < CKPT_PIECES && st == hipSuccess; i++) {
+                    const size_t from = piece_of(i), to = piece_of(i + 1);
+                    st = hipEventSynchronize(on_host[l * CKPT_PIECES + i]);
+                    if (st != hipSuccess) break;
+                    if (hash) sha.blocks(rows + from, (to - from) / 64);  // pieces but the last are whole pages
+                    else std::memcpy((uint8_t*)(out_rows + l * n) + from, rows + from, to - from);
                 }
-                const uint8_t* rows = s->ckpt_host + l * n * 4;
-                if (out_rows) std::memcpy(out_rows + l * n, rows, n * 4);
-                if (out_hashes) iris_sha256(rows, n * 4, out_hashes + 32 * l);
+                if (st != hipSuccess) status = (int)st;
+                else if (hash) sha.finish(rows + bytes / 64 * 64, bytes % 64, out_hashes + 32 * l);
             }
         });
     for (auto& th : pool) th.join();
@@ -1430,6 +1498,15 @@ int iris_session_layer_stage(IrisSession* s, uint32_t layer, const int32_t* in_r
     return rc;
 }
 
+// Every page of a host buffer that a copy will fill, made present while the
+// device works, its contents kept: a fresh buffer's page faults otherwise
+// come one by one inside the copy.
+static void touch_pages(void* p, size_t bytes) {
+    volatile uint8_t* b = (volatile uint8_t*)p;
+    for (size_t i = 0; i < bytes; i += 4096) __atomic_fetch_or(&b[i], 0, __ATOMIC_RELAXED);
+    if (bytes) __atomic_fetch_or(&b[bytes - 1], 0, __ATOMIC_RELAXED);
+}
+
 static int layer_stage_run(IrisSession* s, uint32_t layer, const int32_t* in_rows, uint32_t count,
                            uint32_t start_position, const int32_t* ple_rows, int32_t* out_rows) {
     IrisModel* m = s->model;
@@ -1451,6 +1528,7 @@ static int layer_stage_run(IrisSession* s, uint32_t layer, const int32_t* in_row
         RT_CHECK(iris_rope_table_launch(m->inv_freq, d.head_dim / 2, s->d_pos, count, s->rope_sc, st));
         RT_CHECK(mistral_layer(s, layer, count, false, false));
     }
+    touch_pages(out_rows, (size_t)count * H * 4);
     RT_CHECK(hipMemcpyAsync(out_rows, s->x, (size_t)count * H * 4, hipMemcpyDeviceToHost, st));
     return (int)hipStreamSynchronize(st);
 }

@@ -67,6 +67,8 @@ struct IrisModel {
     bool finalized = false;
 };
 
+constexpr uint32_t CKPT_PIECES = 4, LOGITS_SLOTS = 4;
+
 struct IrisSession {
     IrisModel* model = nullptr;
     uint32_t max_positions = 0, max_rows = 0;
@@ -134,10 +136,26 @@ struct IrisSession {
     int32_t* ckpt_dev = nullptr;              // [layers][max_rows][hidden]
     uint8_t* ckpt_host = nullptr;             // pinned, same shape
     hipStream_t copy_stream = nullptr;
-    std::vector<hipEvent_t> ckpt_events;      // [2][layers]: rows copied on the device, on the host
+    // [layers] rows copied on the device, then [layers][CKPT_PIECES] pieces of them on the host
+    std::vector<hipEvent_t> ckpt_events;
+    // kept logits on their way to the host: LOGITS_SLOTS pinned slots, made
+    // on the first generation that keeps them; per slot, the steps it holds
+    // are made on the device, are in the slot
+    uint8_t* logits_ring = nullptr;
+    size_t logits_slot = 0;  // bytes
+    hipEvent_t logits_events[2 * LOGITS_SLOTS] = {};
     hipGraphExec_t graph_exec = nullptr;
     bool graph_keep_logits = false;
 };
 
-// SHA-256 (FIPS 180-4) of `len` bytes into out[32].
+// SHA-256 (FIPS 180-4): whole 64-byte blocks as they come, then the rest
+// (under 64 bytes).
+struct Sha256 {
+    uint32_t h[8] = {0x6a09e667, 0xbb67ae85, 0x3c6ef372, 0xa54ff53a, 0x510e527f, 0x9b05688c, 0x1f83d9ab, 0x5be0cd19};
+    uint64_t total = 0;
+    void blocks(const uint8_t* data, size_t n);
+    void finish(const uint8_t* data, size_t rem, uint8_t out[32]);
+};
+
+// SHA-256 of `len` bytes into out[32].
 void iris_sha256(const uint8_t* data, size_t len, uint8_t out[32]);

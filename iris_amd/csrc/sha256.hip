@@ -91,16 +91,17 @@ void compress_blocks(uint32_t h[8], const uint8_t* p, size_t blocks) {
 
 }  // namespace
 
-void iris_sha256(const uint8_t* data, size_t len, uint8_t out[32]) {
-    uint32_t h[8] = {0x6a09e667, 0xbb67ae85, 0x3c6ef372, 0xa54ff53a, 0x510e527f, 0x9b05688c, 0x1f83d9ab, 0x5be0cd19};
-    const size_t i = len / 64 * 64;
-    compress_blocks(h, data, len / 64);
+void Sha256::blocks(const uint8_t* data, size_t n) {
+    compress_blocks(h, data, n);
+    total += n * 64;
+}
+
+void Sha256::finish(const uint8_t* data, size_t rem, uint8_t out[32]) {
     uint8_t tail[128] = {0};
-    const size_t rem = len - i;
-    std::memcpy(tail, data + i, rem);
+    if (rem) std::memcpy(tail, data, rem);
     tail[rem] = 0x80;
     const size_t tl = rem + 9 <= 64 ? 64 : 128;
-    const uint64_t bits = (uint64_t)len * 8;
+    const uint64_t bits = (total + rem) * 8;
     for (int k = 0; k < 8; k++) tail[tl - 1 - k] = (uint8_t)(bits >> (8 * k));
     compress_blocks(h, tail, tl / 64);
     for (int k = 0; k < 8; k++) {
@@ -109,6 +110,12 @@ void iris_sha256(const uint8_t* data, size_t len, uint8_t out[32]) {
         out[4 * k + 2] = (uint8_t)(h[k] >> 8);
         out[4 * k + 3] = (uint8_t)h[k];
     }
+}
+
+void iris_sha256(const uint8_t* data, size_t len, uint8_t out[32]) {
+    Sha256 s;
+    s.blocks(data, len / 64);
+    s.finish(data + len / 64 * 64, len % 64, out);
 }
 
 extern "C" int iris_sha256_bytes(const uint8_t* data, uint64_t len, uint8_t* out) {
