@@ -65,10 +65,9 @@ __device__ __forceinline__ int wave_max_int(int v) {
 // Query planes: one wave per (16-row tile, head). Lane l takes row l % 16
 // and dims 16 * (l / 16) .. + 16 of each 64-dim step.
 template <uint32_t HD>
-__global__ __launch_bounds__(64) void attn_q_planes_kernel(const AttnArgs a, uint32_t tokens) {
+__device__ __forceinline__ void q_planes(const AttnArgs& a, uint32_t tokens, uint32_t qt, uint32_t h, uint32_t lane) {
     constexpr uint32_t DS = HD / 64;
     const AttnPlanes& p = a.planes;
-    const uint32_t qt = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
     const uint32_t t = qt * 16 + (lane & 15), dq = (lane >> 4) * 16;
     const bool valid = t < tokens;
     const int32_t* q = a.q + (size_t)(valid ? t : 0) * a.q_stride + (size_t)h * HD;
@@ -100,12 +99,21 @@ __global__ __launch_bounds__(64) void attn_q_planes_kernel(const AttnArgs a, uin
 // l % 16 and dims 16 * (l / 16) .. of each 64-dim step. Value d-tiles
 // w, w + 4, ...: lane l takes dim l % 16 and, as byte 4t + i, the key
 // 16t + 4(l / 16) + i of the step.
+// The launch's first ks_cap * kv_heads workgroups; the rest make the query
+// planes, four (tile, head) pairs each (one launch less, and the queries'
+// short chains run beside the keys': 45 rows after 1500 keys 6 + 16 us -> 18).
 template <uint32_t HD>
-__global__ __launch_bounds__(256) void attn_kv_planes_kernel(const AttnArgs a, uint32_t tokens) {
+__global__ __launch_bounds__(256) void attn_planes_kernel(const AttnArgs a, uint32_t tokens) {
     constexpr uint32_t DS = HD / 64, DT = HD / 16;
     __shared__ int s_need[2];
     const AttnPlanes& p = a.planes;
-    const uint32_t ks = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (blockIdx.x >= p.ks_cap * a.kv_heads) {
+        const uint32_t pair = (blockIdx.x - p.ks_cap * a.kv_heads) * 4 + wave, QT = (tokens + 15) / 16;
+        if (pair < QT * a.heads) q_planes<HD>(a, tokens, pair % QT, pair / QT, lane);
+        return;
+    }
+    const uint32_t ks = blockIdx.x % p.ks_cap, g = blockIdx.x / p.ks_cap;
     const uint32_t nkeys = (uint32_t)(*a.d_pos) + tokens;
     if (ks * 64 >= nkeys) return;
     if (tid < 2) s_need[tid] = 1;
@@ -684,8 +692,8 @@ bool prefill_split(const AttnArgs& a, uint32_t tokens) {
 template <uint32_t HD>
 int prefill_launch(const AttnArgs& a, uint32_t tokens, hipStream_t stream) {
     const uint32_t QT = (tokens + 15) / 16;
-    hipLaunchKernelGGL(attn_q_planes_kernel<HD>, dim3(QT, a.heads), dim3(64), 0, stream, a, tokens);
-    hipLaunchKernelGGL(attn_kv_planes_kernel<HD>, dim3(a.planes.ks_cap, a.kv_heads), dim3(256), 0, stream, a, tokens);
+    hipLaunchKernelGGL(attn_planes_kernel<HD>, dim3(a.planes.ks_cap * a.kv_heads + (QT * a.heads + 3) / 4), dim3(256), 0,
+                       stream, a, tokens);
     const uint32_t wgs = QT * (a.heads / 4);
     if constexpr (HD <= 256) {
         if (prefill_split(a, tokens)) {

@@ -31,26 +31,36 @@
 
 namespace {
 
-// Per token, one wave each, under the rms_norm prologue only: the token's
-// scale (ops.rs:98-114, rms_norm_scale of the order-free saturating sum of
-// squares) at token_limbs[t].
+// Per token, one workgroup each, under the rms_norm prologue only: the
+// token's scale (ops.rs:98-114, rms_norm_scale of the order-free saturating
+// sum of squares) at token_limbs[t]. A launch of few tokens lasts as long as
+// one token's chain, so its row is spread over four waves with four loads in
+// flight per lane (K = 4096: one round; one wave with one load at a time
+// took 9.2 us for 45 tokens and 9.6 for 512, now 4.7 and 5.3).
 __global__ __launch_bounds__(256) void token_prep_kernel(const GemvArgs a) {
-    const uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (t >= a.tokens) return;
-    {
-        const uint32_t K = a.w.cols;
-        const int32_t* x = a.x + (size_t)t * a.x_stride;
-        int64_t s = 0;
-        for (uint32_t k = lane * 4; k < K; k += 256) {
-            const int4 v = *(const int4*)(x + k);
-            s = dn::acc_add_sat(s, (int64_t)v.x * v.x);
-            s = dn::acc_add_sat(s, (int64_t)v.y * v.y);
-            s = dn::acc_add_sat(s, (int64_t)v.z * v.z);
-            s = dn::acc_add_sat(s, (int64_t)v.w * v.w);
+    __shared__ int64_t s_sum[4];
+    const uint32_t t = blockIdx.x, tid = threadIdx.x, K4 = a.w.cols / 4;
+    const int4* x = (const int4*)(a.x + (size_t)t * a.x_stride);
+    int64_t s = 0;
+    for (uint32_t k = tid; k < K4; k += 1024) {
+        int4 v[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) v[u] = x[min(k + 256 * u, K4 - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            if (k + 256 * u >= K4) continue;
+            s = dn::acc_add_sat(s, (int64_t)v[u].x * v[u].x);
+            s = dn::acc_add_sat(s, (int64_t)v[u].y * v[u].y);
+            s = dn::acc_add_sat(s, (int64_t)v[u].z * v[u].z);
+            s = dn::acc_add_sat(s, (int64_t)v[u].w * v[u].w);
         }
-        for (int off = 32; off >= 1; off >>= 1) s = dn::acc_add_sat(s, __shfl_xor(s, off));
-        if (lane == 0) a.token_limbs[t] = dn::rms_scale_from_sum(s, K, a.norm_eps);
     }
+    for (int off = 32; off >= 1; off >>= 1) s = dn::acc_add_sat(s, __shfl_xor(s, off));
+    if (tid % 64 == 0) s_sum[tid / 64] = s;
+    __syncthreads();
+    if (tid) return;
+    for (int i = 1; i < 4; i++) s = dn::acc_add_sat(s, s_sum[i]);
+    a.token_limbs[t] = dn::rms_scale_from_sum(s, a.w.cols, a.norm_eps);
 }
 
 __global__ __launch_bounds__(256) void fill_ints_kernel(int32_t* p, uint32_t n, int32_t v) {
@@ -63,13 +73,22 @@ __global__ __launch_bounds__(256) void fill_ints_kernel(int32_t* p, uint32_t n, 
 // scale), w)), in the operand layout above, and the digits the chunk's
 // values need, stored for the (chunk, tile) at token_limbs[M + chunk * TT +
 // tile]: every launch writes each of its counts, so none needs a reset.
-// Tokens past the end of the last tile get zero digits.
-__global__ __launch_bounds__(256) void digit_planes_kernel(const GemvArgs a) {
+// Tokens past the end of the last tile get zero digits. A launch of few
+// workgroups takes one wave per k block, so that it lasts one load's latency
+// instead of two (K = 4096, us: 45 tokens 8.2 -> 6.4); with many, four waves
+// of two blocks each are faster (2048 tokens, normed: 21.5 against 26.5).
+// The gated rows' counts, which the product's workgroups raise, start at 1:
+// set here (ones of them) for the product that follows.
+constexpr uint32_t DP_THREADS = 64 * PLANE_KB;
+__global__ __launch_bounds__(DP_THREADS) void digit_planes_kernel(const GemvArgs a, uint32_t ones) {
     __shared__ int s_need;
     const uint32_t tt = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t K = a.w.cols, M = a.tokens, TT = (M + 31) / 32, KB = K / 32;
     const uint32_t kb0 = blockIdx.y * PLANE_KB, kb1 = min(kb0 + PLANE_KB, KB);
     const bool norm = a.prologue == PRO_RMSNORM;
+    for (uint32_t i = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + tid; i < ones;
+         i += gridDim.x * gridDim.y * blockDim.x)
+        a.out_gemm_limbs[M + i] = 1;
     if (tid == 0) s_need = 1;
     __syncthreads();
     // Lane l writes the 16 bytes of token l % 32 at k-offset 16 * (l / 32)
@@ -80,7 +99,7 @@ __global__ __launch_bounds__(256) void digit_planes_kernel(const GemvArgs a) {
     const int32_t* x = a.x + (size_t)(valid ? t : 0) * a.x_stride;
     const size_t lstride = (size_t)TT * KB * FRAG;
     int need = 1;
-    for (uint32_t kb = kb0 + wave; kb < kb1; kb += 4) {
+    for (uint32_t kb = kb0 + wave; kb < kb1; kb += blockDim.x / 64) {
         const uint32_t k0 = kb * 32 + q * 16;
         uint32_t out[PL_MAX][4];
 #pragma unroll
@@ -105,7 +124,7 @@ __global__ __launch_bounds__(256) void digit_planes_kernel(const GemvArgs a) {
             *(uint4*)(dst + l * lstride) = make_uint4(out[l][0], out[l][1], out[l][2], out[l][3]);
     }
     for (int off = 32; off >= 1; off >>= 1) need = max(need, __shfl_xor(need, off));
-    if (lane == 0) atomicMax(&s_need, need);  // the largest of four: any order
+    if (lane == 0) atomicMax(&s_need, need);  // the largest of the waves: any order
     __syncthreads();
     if (tid == 0) a.token_limbs[M + blockIdx.y * TT + tt] = s_need;
 }
@@ -134,15 +153,17 @@ int iris_gemm_launch(const GemvArgs& a, hipStream_t stream) {
         return IRIS_E_INVALID;
     if (!a.out && !a.out_gemm_planes) return IRIS_E_INVALID;
     const uint32_t TT = (a.tokens + 31) / 32, KB = a.w.cols / 32;
+    // The gated rows' counts start at 1 (every workgroup raises its own).
+    const uint32_t ones = a.out_gemm_planes ? (uint32_t)(gemm_limb_ints(a.w.rows / 2, a.tokens) - a.tokens) : 0;
     if (!a.planes_ready) {
         if (a.prologue == PRO_RMSNORM)
-            hipLaunchKernelGGL(token_prep_kernel, dim3((a.tokens + 3) / 4), dim3(256), 0, stream, a);
-        hipLaunchKernelGGL(digit_planes_kernel, dim3(TT, (KB + PLANE_KB - 1) / PLANE_KB), dim3(256), 0, stream, a);
-    }
-    if (a.out_gemm_planes) {
-        // The gated rows' counts start at 1 (every workgroup raises its own).
-        const uint32_t n = (uint32_t)(gemm_limb_ints(a.w.rows / 2, a.tokens) - a.tokens);
-        hipLaunchKernelGGL(fill_ints_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, a.out_gemm_limbs + a.tokens, n, 1);
+            hipLaunchKernelGGL(token_prep_kernel, dim3(a.tokens), dim3(256), 0, stream, a);
+        const dim3 grid(TT, (KB + PLANE_KB - 1) / PLANE_KB);
+        const bool few = grid.x * grid.y <= 2 * (uint32_t)iris_device_cus();
+        hipLaunchKernelGGL(digit_planes_kernel, grid, dim3(few ? DP_THREADS : 256), 0, stream, a, ones);
+    } else if (ones) {
+        hipLaunchKernelGGL(fill_ints_kernel, dim3((ones + 255) / 256), dim3(256), 0, stream, a.out_gemm_limbs + a.tokens,
+                           ones, 1);
     }
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return (int)st;
