@@ -25,21 +25,19 @@ __device__ __forceinline__ uint32_t plane_byte4(uint64_t d0, uint64_t d1, uint64
            ((uint32_t)((d3 >> sh) & 0xff) << 24);
 }
 
-// The digits a workgroup's token tiles tt0 .. tt0 + tg - 1 need: the most
-// any k chunk of them needs, from digit_planes_kernel's counts.
-__device__ __forceinline__ int tiles_limbs(const GemvArgs& a, uint32_t tt0, uint32_t tg, int& s_limbs) {
-    const uint32_t tid = threadIdx.x, TT = (a.tokens + 31) / 32;
-    const uint32_t chunks = (a.w.cols / 32 + PLANE_KB - 1) / PLANE_KB;
-    const int32_t* need = a.token_limbs + a.tokens;
-    if (tid == 0) s_limbs = 1;
-    __syncthreads();
-    for (uint32_t i = tid; i < tg * chunks; i += blockDim.x) {
-        const uint32_t t = tt0 + i % tg;
-        if (t < TT) atomicMax(&s_limbs, need[(i / tg) * TT + t]);
-    }
-    __syncthreads();
-    const int limbs = s_limbs;
-    __syncthreads();
+// The digits a workgroup's TG token tiles from tt0 (uniform) need: the most
+// any k chunk of them needs, from digit_planes_kernel's counts. Every wave
+// reads them itself through scalar loads (written by an earlier launch, only
+// read here): no LDS, no barrier, and no wait on the vector loads in flight.
+template <uint32_t TG>
+__device__ __forceinline__ int tiles_limbs(const GemvArgs& a, uint32_t tt0) {
+    const uint32_t TT = (a.tokens + 31) / 32, chunks = (a.w.cols / 32 + PLANE_KB - 1) / PLANE_KB;
+    const auto* need = (const __attribute__((address_space(4))) int32_t*)(uintptr_t)(a.token_limbs + a.tokens);
+    int limbs = 1;
+#pragma unroll 4
+    for (uint32_t c = 0; c < chunks; c++)
+#pragma unroll
+        for (uint32_t t = 0; t < TG; t++) limbs = max(limbs, need[c * TT + min(tt0 + t, TT - 1)]);
     return limbs;
 }
 

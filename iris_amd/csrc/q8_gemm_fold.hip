@@ -243,12 +243,11 @@ __global__ __launch_bounds__(64 * W, 1) void q8_gemm_fold_kernel(const GemvArgs 
     static_assert(FoldShape<WP, 3, W, RT>::TTWG == TG && TG % FoldShape<WP, 5, W, RT>::TTWG == 0, "whole passes");
     constexpr uint32_t S3 = FoldShape<WP, 3, W, RT>::SMEM, S5 = FoldShape<WP, 5, W, RT>::SMEM;
     __shared__ __attribute__((aligned(1024))) int8_t smem[S5 > S3 ? S5 : S3];
-    int& s_limbs = *(int*)smem;
     const uint32_t TT = (a.tokens + 31) / 32;
     uint32_t rg, tg;
     tile_of_block(blockIdx.x, (a.w.tiles + 2 * RT - 1) / (2 * RT), (TT + TG - 1) / TG, rg, tg);
     const uint32_t rt0 = rg * RT, tt0 = tg * TG;
-    const int limbs = tiles_limbs(a, tt0, TG, s_limbs);
+    const int limbs = tiles_limbs<TG>(a, tt0);
     switch (limbs) {
         case 1: fold_pass<WP, 1, W, RT>(a, smem, rt0, tt0); break;
         case 2: fold_pass<WP, 2, W, RT>(a, smem, rt0, tt0); break;

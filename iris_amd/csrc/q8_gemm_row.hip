@@ -227,13 +227,12 @@ __global__ __launch_bounds__(64 * W * SPLIT, 1) void q8_gemm_row_kernel(const Ge
     static_assert(TG == 2 || TG == 4, "64 or 128 tokens per workgroup");
     using G = GemmShape<W, SPLIT>;
     __shared__ __attribute__((aligned(1024))) int8_t smem[G::SMEM];
-    int& s_limbs = *(int*)smem;  // read before the ring is first filled
     const uint32_t TT = (a.tokens + 31) / 32;
     uint32_t rg, tg;
     tile_of_block(blockIdx.x, (a.w.tiles + 2 * G::RT - 1) / (2 * G::RT), (TT + TG - 1) / TG, rg, tg);
     const uint32_t rt0 = rg * G::RT, tt0 = tg * TG;
 
-    const int limbs = tiles_limbs(a, tt0, TG, s_limbs);
+    const int limbs = tiles_limbs<TG>(a, tt0);
     constexpr int RI = TG;  // W waves, one token tile each: W * RI / TG row tiles
     switch (limbs) {
         case 1: gemm_pass<G, 1, RI, DEEP>(a, smem, rt0, tt0); break;

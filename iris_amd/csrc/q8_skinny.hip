@@ -279,7 +279,7 @@ __global__ __launch_bounds__(64 * W, SH == 16 ? 4 : 2) void q8_skinny_kernel(con
     const uint32_t g = blockIdx.x / (8 * tok_tiles), in = blockIdx.x % (8 * tok_tiles);
     const uint32_t rt = g * 8 + in % 8, tt = in / 8;
     if (rt >= row_tiles) return;
-    if (tiles_limbs(a, tt, 1, *(int*)smem) <= 3) skinny_tile<SH, MODE, 3, 4, W>(a, smem, rt, tt);
+    if (tiles_limbs<1>(a, tt) <= 3) skinny_tile<SH, MODE, 3, 4, W>(a, smem, rt, tt);
     else skinny_tile<SH, MODE, 5, 3, W>(a, smem, rt, tt);
 }
 
