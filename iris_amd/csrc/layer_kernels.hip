@@ -440,7 +440,7 @@ __global__ __launch_bounds__(256) void silu_table_kernel(int32_t* tab) {
 __global__ __launch_bounds__(256) void silu_lookup_kernel(const int32_t* tab, const int32_t* x, uint32_t n,
                                                           int32_t* out) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = dn::silu_from_tab(x[i], tab[dn::silu_tab_index(x[i])]);
+    if (i < n) out[i] = dn::silu_quick(x[i], tab);
 }
 
 // The pass position and the selection step of a session, set on its stream.

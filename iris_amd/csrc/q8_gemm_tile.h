@@ -96,20 +96,25 @@ __device__ __forceinline__ void finish_parked(const GemvArgs& a, int32_t* block,
     const bool valid = token < a.tokens && row0 < w.rows;
     const uint32_t n = row0 < w.rows ? min(16u, w.rows - row0) : 0;
     if (a.epilogue == EPI_SWIGLU || a.epilogue == EPI_GEGLU) {
-        // Gate and up rows alternate. silu by table: the eight pairs'
-        // gathers are in flight together.
+        // Gate and up rows alternate.
         int32_t o[8];
         if (a.epilogue == EPI_SWIGLU && a.silu_tab) {
-            int32_t gate[8], up[8], looked[8];
+            int32_t gate[8], up[8], act[8];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const int4 v = *(const int4*)(p + 4 * q);
                 gate[2 * q] = v.x, up[2 * q] = v.y, gate[2 * q + 1] = v.z, up[2 * q + 1] = v.w;
             }
+            uint32_t slow = 0;
 #pragma unroll
-            for (int q = 0; q < 8; q++) looked[q] = a.silu_tab[dn::silu_tab_index(gate[q])];
+            for (int q = 0; q < 8; q++) slow |= (uint32_t)!dn::silu_fast(gate[q], act[q]) << q;
+            if (slow) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) o[q] = dn::mul_sat(dn::silu_from_tab(gate[q], looked[q]), up[q]);
+                for (int q = 0; q < 8; q++)
+                    if ((slow >> q) & 1) act[q] = dn::silu_from_tab(gate[q], a.silu_tab[dn::silu_tab_index(gate[q])]);
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++) o[q] = dn::mul_sat(act[q], up[q]);
         } else {
 #pragma unroll 1
             for (int q = 0; q < 8; q++) {  // in place: pair q is read before slot q is written

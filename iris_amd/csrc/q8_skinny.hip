@@ -226,9 +226,7 @@ __device__ __forceinline__ void skinny_tile(const GemvArgs& a, int32_t* smem, ui
         const uint32_t pl = c % PAIRS, tl = c / PAIRS, pair = row0 / 2 + pl, token = tok0 + tl;
         if (2 * pair >= w.rows || token >= a.tokens) continue;
         const int32_t gate = smem[2 * pl * STRIDE + tl], up = smem[(2 * pl + 1) * STRIDE + tl];
-        const int32_t act = a.epilogue == EPI_GEGLU ? dn::gelu(gate)
-                            : a.silu_tab ? dn::silu_from_tab(gate, a.silu_tab[dn::silu_tab_index(gate)])
-                                         : dn::silu(gate);
+        const int32_t act = a.epilogue == EPI_GEGLU ? dn::gelu(gate) : dn::silu_quick(gate, a.silu_tab);
         const int32_t o = dn::mul_sat(act, up);
         if (a.out) a.out[(size_t)token * a.out_stride + pair] = o;
         smem[2 * pl * STRIDE + tl] = o;
