@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(scope="module")
 def session():
     native.check(native.lib().q8gpu_init(), "q8gpu_init")
-    m = synth.mistral_model(64, 1, 4, 3, 32, 64, 64, seed=5)  # kv rows of 96 values
+    m = synth.mistral_model(64, 1, 6, 3, 32, 64, 64, seed=5)  # kv rows of 96 values
     return Session(DeviceModel(m), 45000, 1)
 
 
