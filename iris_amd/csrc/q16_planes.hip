@@ -66,7 +66,12 @@ int iris_q16_prepare(const int32_t* w, uint32_t rows, uint32_t cols, Q16Planes* 
     // Rows past the matrix in its last tile keep zero digits.
     st = hipMalloc((void**)&planes, 2 * plane_bytes);
     if (st == hipSuccess) st = hipMalloc((void**)&shift, (size_t)tiles * Q8_TILE_ROWS * sizeof(int32_t));
-    if (st == hipSuccess) st = hipMemsetAsync(planes, 0, 2 * plane_bytes, stream);
+    if (st != hipSuccess) {  // no room for the planes: the per-row kernel serves
+        (void)hipGetLastError();
+        (void)hipFree(planes);
+        return 0;
+    }
+    st = hipMemsetAsync(planes, 0, 2 * plane_bytes, stream);
     if (st == hipSuccess) st = hipMemsetAsync(shift, 0, (size_t)tiles * Q8_TILE_ROWS * sizeof(int32_t), stream);
     if (st == hipSuccess) {
         hipLaunchKernelGGL(q16_planes_kernel, dim3((unsigned)((blocks + 255) / 256)), dim3(256), 0, stream, w, rows, nb,
