@@ -22,8 +22,12 @@
 // ((l * TT + tt) * KB + kb) * 1024. Every operand is copied from global
 // memory straight into LDS (global_load_lds_dwordx4: each lane fetches its
 // own 16 bytes, the wave writes one contiguous kilobyte, no registers in
-// between) through a four-deep ring of 64-wide k steps, and read back by
-// each lane as one conflict-free 16-byte LDS load.
+// between) through a ring of 64-wide k steps, and read back by each lane as
+// one conflict-free 16-byte LDS load.
+//
+// This file: the activations' preparation and the dispatch. The tiled
+// products are in q8_gemm_row.hip and q8_gemm_fold.hip, those of few tokens
+// in q8_skinny.hip.
 #include "detnum_dev.h"
 #include "q8_gemm_common.h"
 #include "q8_gemm_row.h"

@@ -16,8 +16,8 @@
 // instructions per 16 weights beside nine matrix instructions.
 //
 // Measured against the tiled GEMM (us per product, preparation included):
-// 4096 x 14336 per-block scales, 13 tokens 225 -> 25 (2.5 TB/s of weights);
-// 6144 x 4096 row scales, 77 tokens 39.6 -> 27.4; 4096 x 4096 per-block, 24
+// 4096 x 14336 per-block scales, 13 tokens 225 -> 23.4 (2.7 TB/s of weights);
+// 6144 x 4096 row scales, 77 tokens 39.6 -> 26.5; 4096 x 4096 per-block, 24
 // tokens 81 -> 22; and where an unfolded per-block matrix went through the
 // one-token kernel once per token, 24 tokens of 4096 x 4096 93 -> 22.
 //
@@ -287,12 +287,12 @@ __global__ __launch_bounds__(64 * W, SH == 16 ? 4 : 2) void q8_skinny_kernel(con
 // few enough rounds of the chip that reading the operands per tile costs less
 // than the GEMM's idle CUs. us, GEMM against this kernel, preparation
 // included, where the rule's bound of four tiles per CU lies:
-//   row scales  4096 x 4096   128 tokens  40.2 / 24.8,   256 tokens  41.6 / 42
-//               28672 x 4096   32 tokens  64.4 / 48,      64 tokens  66.3 / 66
-//               4096 x 14336  128 tokens  97.6 / 51.2,   256 tokens  99.7 / 105
-//   per block   4096 x 4096   128 tokens  83.6 / 35.0,   512 tokens  91.3 / 128
-//               28672 x 4096   32 tokens  91.1 / 66.0,    64 tokens  93.7 / 106
-//               4096 x 14336  128 tokens 228.9 / 90.5,   512 tokens 262.8 / 350
+//   row scales  4096 x 4096   100 tokens  33.5 / 24.6,   200 tokens  37 / 37,   400 tokens  38 / 58
+//               28672 x 4096   45 tokens  54.0 / 54.3,   128 tokens  59 / 93
+//               4096 x 14336   64 tokens   126 / 33.4,   128 tokens  80 / 53,   300 tokens  86 / 119
+//   per block   4096 x 4096   100 tokens  67.1 / 34.8,   200 tokens  70 / 58,   400 tokens  76 / 98
+//               28672 x 4096   45 tokens  84.1 / 101,     64 tokens  88 / 103
+//               4096 x 14336   64 tokens   202 / 52.0,   128 tokens 204 / 90,   300 tokens 215 / 207
 // Up to 16 tokens it always is (28672 x 4096: 62.0 / 41.6 and 89.4 / 48.7).
 static bool few_tiles(const GemvArgs& a) {
     return a.tokens <= 16 ||
