@@ -374,6 +374,10 @@ __device__ __forceinline__ void prefill_wave(const AttnArgs& a, uint32_t tokens,
             }
         }
     }
+    // No key was taken: every visible score is INT32_MIN (a score saturates
+    // there from q.k = -2^50 on at head size 64), and the first of them is
+    // the first maximum.
+    if (best_key == 0xffffffffu) best_key = qstart;
 
     // (2) the sum of exp terms (non-negative, so no order and no saturation)
     // from the stored scores; each lane overwrites a tile's scores with its
