@@ -25,6 +25,7 @@
 #include <thread>
 #include <vector>
 
+#include "checkpoint_jobs.h"
 #include "layer_kernels.h"
 #include "q8_internal.h"
 #include "runtime_internal.h"
@@ -1419,8 +1420,8 @@ static int layer_range_run(IrisSession* s, const int32_t* ids, uint32_t count, u
     RT_CHECK(session_pass(s, count, &sink));
     // A layer's hash is one serial chain over its rows (about 2 GB/s), the
     // longest part of a pass of few layers, so it starts with the first
-    // quarter to arrive and nothing else runs in its thread: the copies into
-    // the caller's rows, with their page faults, are other jobs.
+    // quarter to arrive, and the copy into the caller's rows, with its page
+    // faults, is a job of its own.
     const size_t bytes = n * 4, piece = (bytes / CKPT_PIECES + 4095) / 4096 * 4096;
     auto piece_of = [&](uint32_t i) { return std::min(bytes, i * piece); };
     for (uint32_t l = 0; l < layers; l++) {
@@ -1434,31 +1435,21 @@ static int layer_range_run(IrisSession* s, const int32_t* ids, uint32_t count, u
         }
     }
     const unsigned hw = std::thread::hardware_concurrency();
-    const uint32_t jobs = 2 * layers;  // even: a layer's hash, odd: its rows
-    const uint32_t workers = std::max(1u, std::min({jobs, 16u, hw ? hw : 1u}));
     std::atomic<int> status{0};
-    std::vector<std::thread> pool;
-    for (uint32_t t = 0; t < workers; t++)
-        pool.emplace_back([&, t] {
-            for (uint32_t job = t; job < jobs; job += workers) {
-                const uint32_t l = job / 2;
-                const bool hash = job % 2 == 0;
-                if (hash ? !out_hashes : !out_rows) continue;
-                const uint8_t* rows = s->ckpt_host + l * bytes;
-                Sha256 sha;
-                hipError_t st = hipSuccess;
-                for (uint32_t i = 0; i < CKPT_PIECES && st == hipSuccess; i++) {
-                    const size_t from = piece_of(i), to = piece_of(i + 1);
-                    st = hipEventSynchronize(on_host[l * CKPT_PIECES + i]);
-                    if (st != hipSuccess) break;
-                    if (hash) sha.blocks(rows + from, (to - from) / 64);  // pieces but the last are whole pages
-                    else std::memcpy((uint8_t*)(out_rows + l * n) + from, rows + from, to - from);
-                }
-                if (st != hipSuccess) status = (int)st;
-                else if (hash) sha.finish(rows + bytes / 64 * 64, bytes % 64, out_hashes + 32 * l);
-            }
-        });
-    for (auto& th : pool) th.join();
+    run_checkpoint_jobs(layers, out_hashes, out_rows, std::min(16u, hw), [&](uint32_t l, bool hash) {
+        const uint8_t* rows = s->ckpt_host + l * bytes;
+        Sha256 sha;
+        hipError_t st = hipSuccess;
+        for (uint32_t i = 0; i < CKPT_PIECES && st == hipSuccess; i++) {
+            const size_t from = piece_of(i), to = piece_of(i + 1);
+            st = hipEventSynchronize(on_host[l * CKPT_PIECES + i]);
+            if (st != hipSuccess) break;
+            if (hash) sha.blocks(rows + from, (to - from) / 64);  // pieces but the last are whole pages
+            else std::memcpy((uint8_t*)(out_rows + l * n) + from, rows + from, to - from);
+        }
+        if (st != hipSuccess) status = (int)st;
+        else if (hash) sha.finish(rows + bytes / 64 * 64, bytes % 64, out_hashes + 32 * l);
+    });
     RT_CHECK(hipStreamSynchronize(s->stream));
     return status;
 }
