@@ -93,8 +93,8 @@ int q8gpu_product_device_ws(const Q8GpuMatrix* matrix, const int32_t* d_activati
  * scales folds: 1 to Q8_FOLD_MAX_PLANES (6) planes, by how far a row's
  * scales spread (3 for the reference bundles' layout, 6 for a subnormal
  * block beside exponent 30). Allocates that many x rows x cols bytes more
- * device memory, plus 4 bytes per row (reported by q8gpu_matrix_info's
- * bytes), and synchronises `stream`. Does nothing, and returns 0, for a
+ * device memory (reported by q8gpu_matrix_info's bytes; rows padded to a
+ * multiple of 16), and synchronises `stream`. Does nothing, and returns 0, for a
  * row-scale matrix or one already prepared. Not to be called while other
  * calls use the matrix. No counterpart in the reference (whose device cache budgets
  * rows*cols + blocks*8 bytes per matrix, gpu.rs:171-173: a prepared matrix

@@ -150,7 +150,7 @@ int iris_q8_upload_parts(const uint8_t* const* parts, const uint32_t* part_rows,
     } else {
         hipFree(m->row_scale);
         m->row_scale = nullptr;
-        m->device_bytes = qs_bytes + sc_bytes;
+        m->device_bytes = qs_bytes + sc_bytes + (size_t)m->tiles * Q8_TILE_ROWS * sizeof(int32_t);  // and fold.shift
     }
     *out = m;
     return 0;

@@ -326,7 +326,7 @@ int iris_q8_prepare_fold(Q8GpuMatrix* m, hipStream_t stream) {
         if (st == hipSuccess) st = hipStreamSynchronize(stream);
         if (st == hipSuccess) {
             m->fold.nplanes = (uint32_t)need;
-            m->device_bytes += plane_bytes * need + (size_t)m->tiles * Q8_TILE_ROWS * sizeof(int32_t);
+            m->device_bytes += plane_bytes * need;
             return 0;
         }
     }

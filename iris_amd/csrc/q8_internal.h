@@ -60,8 +60,7 @@ struct Q8GpuMatrix {
     uint64_t device_bytes;
     // Per-block f16 scales: fold.shift (R per row) and a bound on the digits
     // of the row's w' (from the scales alone, for weights of either extreme)
-    // come with the upload; the planes only with iris_q8_prepare_fold. (The
-    // reported device_bytes count the shifts with the planes.)
+    // come with the upload; the planes only with iris_q8_prepare_fold.
     Q8Folded fold;
     uint32_t digits_bound;
     bool fold_tried;  // the folding was attempted (prepared or refused)

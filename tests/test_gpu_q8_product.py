@@ -311,19 +311,21 @@ def test_per_block_scales_on_the_matrix_cores(kind, planes, tokens, rows, cols):
     m = Q8Matrix.from_bytes(raw, rows, cols)
     assert m.info()["scale_mode"] == "f16"
     before = m.info()["bytes"]
+    # One byte per weight, an f16 per block and a 32-bit shift per row (rows
+    # padded to whole 16-row tiles).
+    padded = (rows + 15) // 16 * 16
+    assert before == padded * (cols + cols // 32 * 2 + 4)
     x = grouped_activations(rng, tokens, cols)
     want = cpu.linear_q8(x, raw)
     # Unprepared: the vector path, and the product allocates nothing.
     assert np.array_equal(product_ws(m, x), want)
     assert m.info()["bytes"] == before
     m.prepare_matrix_cores()
-    # The folded planes were built: one byte per weight per plane (rows
-    # padded to whole 16-row tiles), plus one 32-bit shift per row.
-    tiles = (rows + 15) // 16
-    extra = m.info()["bytes"] - before - tiles * 16 * 4
-    assert extra > 0 and extra % (tiles * 16 * cols) == 0
+    # The folded planes were built: one byte per weight per plane.
+    extra = m.info()["bytes"] - before
+    assert extra > 0 and extra % (padded * cols) == 0
     if planes is not None:
-        assert extra // (tiles * 16 * cols) == planes
+        assert extra // (padded * cols) == planes
     got = product_ws(m, x)
     assert np.array_equal(got, want)
     # again, from the folded planes already there
