@@ -241,7 +241,8 @@ int iris_model_set_tensor(IrisModel* model, const char* name, int32_t width, con
 /* Checks every tensor arrived and finishes the upload. */
 int iris_model_finalize(IrisModel* model);
 void iris_model_free(IrisModel* model);
-/* Device bytes held by the model's weights. */
+/* Device bytes held by the model's matrices, the digit planes that the first
+ * session of more than one row adds to them included. */
 uint64_t iris_model_device_bytes(const IrisModel* model);
 
 /* A KV cache for positions 0..max_positions and work space for passes of up

@@ -86,6 +86,7 @@ int iris_q16_prepare(const int32_t* w, uint32_t rows, uint32_t cols, Q16Planes* 
     }
     p->planes = planes;
     p->shift = shift;
+    p->device_bytes = 2 * plane_bytes + (uint64_t)tiles * Q8_TILE_ROWS * sizeof(int32_t);
     return 0;
 }
 

@@ -74,6 +74,7 @@ struct Q8GpuMatrix {
 struct Q16Planes {
     int8_t* planes = nullptr;  // null: not built (wider values, or a width the tiles do not take)
     int32_t* shift = nullptr;  // [tiles * 16], 8
+    uint64_t device_bytes = 0;
     bool tried = false;
 };
 // Builds p from w [rows][cols] in device memory (once; 2 bytes per value).

@@ -391,6 +391,8 @@ uint64_t iris_model_device_bytes(const IrisModel* m) {
     if (m->d.family == IRIS_FAMILY_GEMMA_DENSE) {
         const uint64_t hp = (uint64_t)m->d.hidden * m->d.ple_width * 4;
         b += (uint64_t)m->layers.size() * 2 * hp + (uint64_t)m->d.layers * hp;  // PLE matrices
+        b += m->ple_model_planes.device_bytes;
+        for (const auto& L : m->layers) b += L.ple_gate_planes.device_bytes + L.ple_proj_planes.device_bytes;
     }
     return b;
 }

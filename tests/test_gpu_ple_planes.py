@@ -38,3 +38,22 @@ def test_ple_projections(kind, ple, rows):
     _, want = cpu.OracleRun(m, rows).pass_rows(list(ids), 0, keep_layers=True)
     for layer in range(m.num_layers):
         assert np.array_equal(got[layer], want[layer]), layer
+
+
+def test_model_device_bytes_count_the_planes():
+    # Two planes of one byte per value and a 32-bit shift per row, rows padded
+    # to whole 16-row tiles, for each of the three kinds of matrix; weights
+    # that need a third digit get none.
+    shape = synth.gemma_shape(256, 2, 4, 1, 64, 512, 64, softcap=30.0)
+    for wide in (False, True):
+        m = synth.gemma_model(shape, 512, seed=2)
+        if wide:
+            m.tensors[synth.PREFIX + "layers.1.per_layer_input_gate.weight"].flat[5] = 1 << 20
+        dm = DeviceModel(m)
+        before = dm.device_bytes()
+        Session(dm, 8, 1)
+        assert dm.device_bytes() == before
+        Session(dm, 8, 8)
+        planes = lambda rows, cols: rows * (2 * cols + 4)
+        want = planes(2 * 64, 256) + 2 * planes(256, 64) + (1 if wide else 2) * planes(64, 256)
+        assert dm.device_bytes() == before + want
