@@ -1552,6 +1552,7 @@ int iris_session_write_kv(IrisSession* s, uint32_t layer, uint32_t pos0, uint32_
     if ((uint64_t)pos0 + count > s->max_positions) return IRIS_E_RANGE;
     if (count == 0) return 0;
     const size_t kvw = s->model->layers[layer].kv_rows;
+    std::lock_guard<std::mutex> guard(s->kv_stage_lock);
     uint32_t chunk = 0;
     RT_CHECK(ensure_kv_stage(s, kvw, count, &chunk));
     for (uint32_t p = 0; p < count; p += chunk) {
@@ -1578,6 +1579,7 @@ int iris_session_read_kv(IrisSession* s, uint32_t layer, uint32_t pos0, uint32_t
     if ((uint64_t)pos0 + count > s->max_positions) return IRIS_E_RANGE;
     if (count == 0) return 0;
     const size_t kvw = s->model->layers[layer].kv_rows;
+    std::lock_guard<std::mutex> guard(s->kv_stage_lock);
     uint32_t chunk = 0;
     RT_CHECK(ensure_kv_stage(s, kvw, count, &chunk));
     for (uint32_t p = 0; p < count; p += chunk) {

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -128,8 +129,10 @@ struct IrisSession {
     int64_t* rope_sc = nullptr;      // mistral-dense: [max_rows][head_dim/2][sin, cos] of the pass's positions
     // multi-row attention digit planes (null for single-row sessions)
     AttnPlanes attn_planes{};
-    // K rows on their way to or from the host (kv_stage_chunk positions at
-    // most), made on the first iris_session_read_kv / write_kv
+    // K rows on their way to or from the host (16 MB or one position at most),
+    // made on the first iris_session_read_kv / write_kv; one call at a time
+    // (reads of one session's caches may come from several threads)
+    std::mutex kv_stage_lock;
     int32_t* kv_stage = nullptr;
     size_t kv_stage_cap = 0;  // ints
     // per-layer checkpoint staging, made on the first checkpointing pass
