@@ -102,6 +102,7 @@ extern "C" {
         scale_mode: *mut c_int,
         bytes: *mut u64,
     ) -> c_int;
+    pub fn iris_product_route(matrix: *const Q8GpuMatrix, tokens: u32, name: *mut c_char, size: u32) -> c_int;
     pub fn q8gpu_synchronize() -> c_int;
 
     pub fn iris_device_malloc(bytes: u64, out: *mut *mut c_void) -> c_int;

@@ -122,6 +122,14 @@ int q8gpu_product_device_noalloc(const Q8GpuMatrix* matrix, const int32_t* d_act
 int q8gpu_matrix_info(const Q8GpuMatrix* matrix, uint32_t* rows, uint32_t* cols, int* scale_mode,
                       uint64_t* bytes);
 
+/* Test query: the kernel shape a `tokens`-token product of the matrix takes
+ * when it is given work space, as text of less than `size` bytes in `name`:
+ * "few SxS, W waves" (tiles of S rows and tokens, their k steps shared by W
+ * waves), "tiled RxT", with " split" (two k groups) and " deep" (deeper
+ * rings), "folded RxT, P planes", or "per token" (the vector kernels). No
+ * counterpart in the reference. */
+int iris_product_route(const Q8GpuMatrix* matrix, uint32_t tokens, char* name, uint32_t size);
+
 /* Waits for all work on the device. */
 int q8gpu_synchronize(void);
 

@@ -1,6 +1,7 @@
 // Host side of the Q8_0 product ABI: matrix upload (raw Q8_0 rows, or the
 // reference's de-interleaved weights + i64 scales), the synchronous drop-in
 // product and the device-pointer product.
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -358,6 +359,19 @@ int q8gpu_matrix_info(const Q8GpuMatrix* m, uint32_t* rows, uint32_t* cols, int*
     if (cols) *cols = m->cols;
     if (scale_mode) *scale_mode = m->scale_mode;
     if (bytes) *bytes = m->device_bytes;
+    return 0;
+}
+
+int iris_product_route(const Q8GpuMatrix* m, uint32_t tokens, char* name, uint32_t size) {
+    if (!m || !name || size == 0) return IRIS_E_INVALID;
+    GemvArgs a{};
+    a.w = q8_view(m);
+    a.tokens = tokens;
+    a.epilogue = EPI_STORE;
+    a.planes = (int8_t*)256;  // aligned, never read
+    a.token_limbs = (int32_t*)256;
+    if (iris_gemm_applies(a)) iris_gemm_route(a, name, size);
+    else std::snprintf(name, size, "per token");
     return 0;
 }
 

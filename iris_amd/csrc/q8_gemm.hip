@@ -174,3 +174,9 @@ int iris_gemm_launch(const GemvArgs& a, hipStream_t stream) {
     if (iris_skinny_applies(a)) return iris_skinny_launch(a, stream);
     return a.w.scale_mode == Q8_SCALE_F16 ? iris_gemm_fold_launch(a, stream) : iris_gemm_row_launch(a, stream);
 }
+
+void iris_gemm_route(const GemvArgs& a, char* name, size_t size) {
+    if (iris_skinny_applies(a)) iris_skinny_route(a, name, size);
+    else if (a.w.scale_mode == Q8_SCALE_F16) iris_gemm_fold_route(a, name, size);
+    else iris_gemm_row_route(a, name, size);
+}

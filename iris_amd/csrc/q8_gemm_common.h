@@ -44,3 +44,4 @@ __device__ __forceinline__ int tiles_limbs(const GemvArgs& a, uint32_t tt0) {
 // Products of few tokens (q8_skinny.hip), their digit planes already made.
 bool iris_skinny_applies(const GemvArgs& a);
 int iris_skinny_launch(const GemvArgs& a, hipStream_t stream);
+void iris_skinny_route(const GemvArgs& a, char* name, size_t size);

@@ -1,4 +1,5 @@
 // The tiled product of per-block scale matrices and the folding it needs.
+#include <cstdio>
 #include <mutex>
 
 #include "q8_gemm_row.h"
@@ -271,28 +272,44 @@ __global__ __launch_bounds__(64 * W, 1) void q8_gemm_fold_kernel(const GemvArgs 
 
 }  // namespace
 
-int iris_gemm_fold_launch(const GemvArgs& a, hipStream_t stream) {
+// The shape of a launch (FoldShape) and its workgroups.
+struct FoldLaunch {
+    uint32_t rows, tokens, blocks;
+};
+
+static FoldLaunch fold_shape(const GemvArgs& a) {
     const uint32_t TT = (a.tokens + 31) / 32, cus = (uint32_t)iris_device_cus();
+    if (a.w.fold_nplanes > 3) return {64, 64, (a.w.tiles + 3) / 4 * ((TT + 1) / 2)};
     const uint32_t rg = (a.w.tiles + 7) / 8, n4 = rg * ((TT + 3) / 4), n2 = rg * ((TT + 1) / 2);
-    const uint32_t n64 = (a.w.tiles + 3) / 4 * ((TT + 1) / 2);
     // A 128-token workgroup takes about 8/5 of a 64-token one's time. us per
     // product, preparation included, 128 / 64 tokens, rows x K:
     //   2048 tokens  28672 x 4096  1637 / 1923    4096 x 14336  841 / 959
     //    512 tokens  28672 x 4096   455 / 514     4096 x 14336  327 / 245
     //    128 tokens  28672 x 4096   141 / 158     512 tokens, 4096 x 4096  104 / 78
-    const bool wide = 8 * ((n4 + cus - 1) / cus) <= 5 * ((n2 + cus - 1) / cus);
+    const bool wide = a.w.fold_nplanes == 3 && 8 * ((n4 + cus - 1) / cus) <= 5 * ((n2 + cus - 1) / cus);
+    return wide ? FoldLaunch{128, 128, n4} : FoldLaunch{128, 64, n2};
+}
+
+int iris_gemm_fold_launch(const GemvArgs& a, hipStream_t stream) {
+    const FoldLaunch s = fold_shape(a);
+    const dim3 grid(s.blocks);
     switch (a.w.fold_nplanes) {
-        case 1: hipLaunchKernelGGL((q8_gemm_fold_kernel<1, 4, 4, 2>), dim3(n2), dim3(256), 0, stream, a); break;
-        case 2: hipLaunchKernelGGL((q8_gemm_fold_kernel<2, 4, 4, 2>), dim3(n2), dim3(256), 0, stream, a); break;
+        case 1: hipLaunchKernelGGL((q8_gemm_fold_kernel<1, 4, 4, 2>), grid, dim3(256), 0, stream, a); break;
+        case 2: hipLaunchKernelGGL((q8_gemm_fold_kernel<2, 4, 4, 2>), grid, dim3(256), 0, stream, a); break;
         case 3:
-            if (wide) hipLaunchKernelGGL((q8_gemm_fold_kernel<3, 8, 4, 4>), dim3(n4), dim3(512), 0, stream, a);
-            else hipLaunchKernelGGL((q8_gemm_fold_kernel<3, 4, 4, 2>), dim3(n2), dim3(256), 0, stream, a);
+            if (s.tokens == 128) hipLaunchKernelGGL((q8_gemm_fold_kernel<3, 8, 4, 4>), grid, dim3(512), 0, stream, a);
+            else hipLaunchKernelGGL((q8_gemm_fold_kernel<3, 4, 4, 2>), grid, dim3(256), 0, stream, a);
             break;
-        case 4: hipLaunchKernelGGL((q8_gemm_fold_kernel<4, 4, 2, 2>), dim3(n64), dim3(256), 0, stream, a); break;
-        case 5: hipLaunchKernelGGL((q8_gemm_fold_kernel<5, 4, 2, 2>), dim3(n64), dim3(256), 0, stream, a); break;
-        default: hipLaunchKernelGGL((q8_gemm_fold_kernel<6, 4, 2, 2>), dim3(n64), dim3(256), 0, stream, a); break;
+        case 4: hipLaunchKernelGGL((q8_gemm_fold_kernel<4, 4, 2, 2>), grid, dim3(256), 0, stream, a); break;
+        case 5: hipLaunchKernelGGL((q8_gemm_fold_kernel<5, 4, 2, 2>), grid, dim3(256), 0, stream, a); break;
+        default: hipLaunchKernelGGL((q8_gemm_fold_kernel<6, 4, 2, 2>), grid, dim3(256), 0, stream, a); break;
     }
     return (int)hipGetLastError();
+}
+
+void iris_gemm_fold_route(const GemvArgs& a, char* name, size_t size) {
+    const FoldLaunch s = fold_shape(a);
+    std::snprintf(name, size, "folded %ux%u, %u planes", s.rows, s.tokens, a.w.fold_nplanes);
 }
 
 int iris_q8_prepare_fold(Q8GpuMatrix* m, hipStream_t stream) {

@@ -1,5 +1,7 @@
 // The tiled product of row-scale matrices (q8_gemm.hip has the arithmetic,
 // the operand layout and the launch rule).
+#include <cstdio>
+
 #include "q8_gemm_row.h"
 #include "q8_gemm_tile.h"
 
@@ -257,7 +259,15 @@ __global__ __launch_bounds__(64 * W * SPLIT, 1) void q8_gemm_row_kernel(const Ge
 
 }  // namespace
 
-int iris_gemm_row_launch(const GemvArgs& a, hipStream_t stream) {
+// The shape of a launch: `waves` per k group over 32 * waves rows, `tokens`
+// tokens, the k steps split between two groups, deep rings, and its workgroups.
+struct RowShape {
+    uint32_t waves, tokens;
+    bool split, deep;
+    uint32_t blocks;
+};
+
+static RowShape row_shape(const GemvArgs& a) {
     const uint32_t TT = (a.tokens + 31) / 32;
     // The shape whose rounds of workgroups cost least: 256 rows x 128 tokens
     // with two waves per SIMD, or 128 x 128 or 128 x 64 with the k steps
@@ -281,16 +291,29 @@ int iris_gemm_row_launch(const GemvArgs& a, hipStream_t stream) {
     const bool split = (a.w.cols / 64) % 2 == 0;
     // Deeper rings for long rows (at least 64 k steps per wave group).
     const bool deep = a.w.cols >= 8192;
-    if (split ? cost8 <= (cost4 < cost2 ? cost4 : cost2) : n8 >= cus)
-        hipLaunchKernelGGL((q8_gemm_row_kernel<8, 4>), dim3(n8), dim3(512), 0, stream, a);
-    else if (n42 != n4 && cost2 <= cost4) {
-        if (split && deep) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2, 2, true>), dim3(n42), dim3(512), 0, stream, a);
-        else if (split) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2, 2>), dim3(n42), dim3(512), 0, stream, a);
-        else hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2>), dim3(n42), dim3(256), 0, stream, a);
+    if (split ? cost8 <= (cost4 < cost2 ? cost4 : cost2) : n8 >= cus) return {8, 128, false, false, n8};
+    if (n42 != n4 && cost2 <= cost4) return {4, 64, split, split && deep, n42};
+    return {4, 128, split, split && deep, n4};
+}
+
+int iris_gemm_row_launch(const GemvArgs& a, hipStream_t stream) {
+    const RowShape s = row_shape(a);
+    const dim3 grid(s.blocks);
+    if (s.waves == 8)
+        hipLaunchKernelGGL((q8_gemm_row_kernel<8, 4>), grid, dim3(512), 0, stream, a);
+    else if (s.tokens == 64) {
+        if (s.deep) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2, 2, true>), grid, dim3(512), 0, stream, a);
+        else if (s.split) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2, 2>), grid, dim3(512), 0, stream, a);
+        else hipLaunchKernelGGL((q8_gemm_row_kernel<4, 2>), grid, dim3(256), 0, stream, a);
     } else {
-        if (split && deep) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 4, 2, true>), dim3(n4), dim3(512), 0, stream, a);
-        else if (split) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 4, 2>), dim3(n4), dim3(512), 0, stream, a);
-        else hipLaunchKernelGGL((q8_gemm_row_kernel<4, 4>), dim3(n4), dim3(256), 0, stream, a);
+        if (s.deep) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 4, 2, true>), grid, dim3(512), 0, stream, a);
+        else if (s.split) hipLaunchKernelGGL((q8_gemm_row_kernel<4, 4, 2>), grid, dim3(512), 0, stream, a);
+        else hipLaunchKernelGGL((q8_gemm_row_kernel<4, 4>), grid, dim3(256), 0, stream, a);
     }
     return (int)hipGetLastError();
+}
+
+void iris_gemm_row_route(const GemvArgs& a, char* name, size_t size) {
+    const RowShape s = row_shape(a);
+    std::snprintf(name, size, "tiled %ux%u%s%s", 32 * s.waves, s.tokens, s.split ? " split" : "", s.deep ? " deep" : "");
 }

@@ -270,6 +270,8 @@ inline uint64_t gemm_limb_ints(uint32_t cols, uint32_t tokens) {
 // returns IRIS_E_INVALID when the launch does not qualify.
 int iris_gemm_launch(const GemvArgs& a, hipStream_t stream);
 bool iris_gemm_applies(const GemvArgs& a);
+// The kernel shape iris_gemm_launch takes, by name.
+void iris_gemm_route(const GemvArgs& a, char* name, size_t size);
 
 // After an EPI_HEAD_SELECT product with the same arguments: selects the first
 // maximum over the tile partials, writes the token, embeds it as the next

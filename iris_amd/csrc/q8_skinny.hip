@@ -34,6 +34,7 @@
 // stream (28672 x 4096, 16 tokens: 58 -> 42 us with eight waves -> four).
 // Four k steps in flight per wave: six hold the 16-row shape at 139
 // registers and one workgroup per CU, five spill its per-block form.
+#include <cstdio>
 #include <type_traits>
 
 #include "detnum_dev.h"
@@ -285,18 +286,28 @@ __global__ __launch_bounds__(64 * W, SH == 16 ? 4 : 2) void q8_skinny_kernel(con
 
 // Whether a product the tiled GEMM takes too is faster here: its tiles make
 // few enough rounds of the chip that reading the operands per tile costs less
-// than the GEMM's idle CUs. us, GEMM against this kernel, preparation
-// included, where the rule's bound of four tiles per CU lies:
-//   row scales  4096 x 4096   100 tokens  33.5 / 24.6,   200 tokens  37 / 37,   400 tokens  38 / 58
-//               28672 x 4096   45 tokens  54.0 / 54.3,   128 tokens  59 / 93
-//               4096 x 14336   64 tokens   126 / 33.4,   128 tokens  80 / 53,   300 tokens  86 / 119
-//   per block   4096 x 4096   100 tokens  67.1 / 34.8,   200 tokens  70 / 58,   400 tokens  76 / 98
-//               28672 x 4096   45 tokens  84.1 / 101,     64 tokens  88 / 103
-//               4096 x 14336   64 tokens   202 / 52.0,   128 tokens 204 / 90,   300 tokens 215 / 207
-// Up to 16 tokens it always is (28672 x 4096: 62.0 / 41.6 and 89.4 / 48.7).
+// than the GEMM's idle CUs, and with per-block scales than its three bytes a
+// weight. Up to 16 tokens it always is (28672 x 4096: 62.0 / 41.6 row scales
+// and 89.4 / 48.7 per block); beyond, us of the GEMM / this kernel,
+// preparation included, matrices rotated through more than the last cache,
+// at tokens (tiles per CU) around where they cross:
+//   row scales  4096 x 4096   192 (3.0)  33.4 / 29.7    224 (3.5)  34.2 / 35.0    256 (4.0)  34.1 / 36.4
+//               4096 x 14336  160 (2.5)  85.8 / 87.3    192 (3.0)  89.6 / 87.6    224 (3.5)  88.2 / 105.5
+//               6144 x 4096   128 (3.0)  39.8 / 34.1    160 (3.8)  40.4 / 39.7    192 (4.5)  40.5 / 45.6
+//               2048 x 2048   384 (3.0)  23.9 / 22.4    448 (3.5)  25.0 / 27.1
+//               16384 x 2048   64 (4.0)  34.7 / 29.3     96 (6.0)  26.9 / 35.8
+//               28672 x 4096   32 (3.5)  63.4 / 48.6     64 (7.0)  59.6 / 67.1
+//   per block   4096 x 4096   320 (5.0)  71.5 / 70.8    384 (6.0)  80.3 / 81.5
+//               4096 x 14336  320 (5.0) 227.7 / 201.5   384 (6.0) 231.8 / 236.1
+//               6144 x 4096   192 (4.5)  69.9 / 68.0    224 (5.3)  75.3 / 76.4
+//               16384 x 2048   64 (4.0)  41.9 / 37.4     96 (6.0)  47.5 / 50.1
+//               28672 x 4096   32 (3.5)  95.1 / 58.5     64 (7.0)  90.4 / 95.6
+// (Up to 64 tokens the GEMM's narrowest workgroup is one token group, partly
+// empty, so row scales cross later there.)
 static bool few_tiles(const GemvArgs& a) {
+    const uint32_t per_cu = a.w.scale_mode == Q8_SCALE_F16 ? 5 : a.tokens <= 64 ? 4 : 3;
     return a.tokens <= 16 ||
-           (uint64_t)((a.w.tiles + 1) / 2) * ((a.tokens + 31) / 32) <= 4ull * (uint32_t)iris_device_cus();
+           (uint64_t)((a.w.tiles + 1) / 2) * ((a.tokens + 31) / 32) <= (uint64_t)per_cu * (uint32_t)iris_device_cus();
 }
 
 bool iris_skinny_applies(const GemvArgs& a) {
@@ -316,9 +327,21 @@ bool iris_skinny_applies(const GemvArgs& a) {
            a.w.cols <= 16384 && (few_tiles(a) || !a.w.fold_planes);
 }
 
-int iris_skinny_launch(const GemvArgs& a, hipStream_t stream) {
+// The shape of a launch: tiles of 16 or 32 rows and tokens, and the waves
+// that share one's k steps.
+struct SkinnyLaunch {
+    uint32_t side, waves, row_tiles, tok_tiles;
+};
+
+static SkinnyLaunch skinny_shape(const GemvArgs& a) {
     const bool small = a.tokens <= 16;
     const uint32_t row_tiles = small ? a.w.tiles : (a.w.tiles + 1) / 2, tok_tiles = (a.tokens + 31) / 32;
+    return {small ? 16u : 32u, row_tiles * tok_tiles <= (uint32_t)iris_device_cus() ? 8u : 4u, row_tiles, tok_tiles};
+}
+
+int iris_skinny_launch(const GemvArgs& a, hipStream_t stream) {
+    const SkinnyLaunch s = skinny_shape(a);
+    const uint32_t row_tiles = s.row_tiles, tok_tiles = s.tok_tiles;
     const dim3 grid((row_tiles + 7) / 8 * 8 * tok_tiles);
     auto launch = [&](auto sh, auto w) {
         constexpr int SH = decltype(sh)::value;
@@ -331,10 +354,14 @@ int iris_skinny_launch(const GemvArgs& a, hipStream_t stream) {
             hipLaunchKernelGGL((q8_skinny_kernel<SH, Q8_SCALE_F16, W>), grid, dim3(64 * W), 0, stream, a, row_tiles, tok_tiles);
     };
     using std::integral_constant;
-    const bool few = row_tiles * tok_tiles <= (uint32_t)iris_device_cus();
-    if (small && few) launch(integral_constant<int, 16>{}, integral_constant<uint32_t, 8>{});
-    else if (small) launch(integral_constant<int, 16>{}, integral_constant<uint32_t, 4>{});
-    else if (few) launch(integral_constant<int, 32>{}, integral_constant<uint32_t, 8>{});
+    if (s.side == 16 && s.waves == 8) launch(integral_constant<int, 16>{}, integral_constant<uint32_t, 8>{});
+    else if (s.side == 16) launch(integral_constant<int, 16>{}, integral_constant<uint32_t, 4>{});
+    else if (s.waves == 8) launch(integral_constant<int, 32>{}, integral_constant<uint32_t, 8>{});
     else launch(integral_constant<int, 32>{}, integral_constant<uint32_t, 4>{});
     return (int)hipGetLastError();
+}
+
+void iris_skinny_route(const GemvArgs& a, char* name, size_t size) {
+    const SkinnyLaunch s = skinny_shape(a);
+    std::snprintf(name, size, "few %ux%u, %u waves", s.side, s.side, s.waves);
 }

@@ -65,6 +65,7 @@ def _declare(L):
         "q8gpu_product_device_noalloc": (C.c_int, [vp, vp, u32, vp, vp]),
         "q8gpu_prepare_matrix_cores": (C.c_int, [vp, vp]),
         "q8gpu_matrix_info": (C.c_int, [vp, C.POINTER(u32), C.POINTER(u32), C.POINTER(C.c_int), C.POINTER(u64)]),
+        "iris_product_route": (C.c_int, [vp, u32, C.c_char_p, u32]),
         "q8gpu_synchronize": (C.c_int, []),
         "iris_device_malloc": (C.c_int, [u64, pp]),
         "iris_device_free": (C.c_int, [vp]),

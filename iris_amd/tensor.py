@@ -64,6 +64,13 @@ class Q8Matrix:
                      "matrix info")
         return {"rows": r.value, "cols": c.value, "scale_mode": SCALE_MODES[mode.value], "bytes": b.value}
 
+    def route(self, tokens: int) -> str:
+        """The kernel shape a ``tokens``-token product with work space takes,
+        by name (include/iris_hip.h, iris_product_route): for tests."""
+        name = C.create_string_buffer(64)
+        native.check(native.lib().iris_product_route(self._h, tokens, name, len(name)), "product route")
+        return name.value.decode()
+
     def free(self):
         if self._h:
             native.lib().q8gpu_free(self._h)

@@ -36,3 +36,18 @@ def test_few_token_products(tokens, rows, cols, kind):
         if bits < 32:
             x = np.clip(x, -(1 << (bits - 1)), (1 << (bits - 1)) - 1).astype(np.int32)
         assert np.array_equal(product_ws(m, x), cpu.linear_q8(x, raw))
+
+
+# Where the tiled GEMM takes over: past three tiles of 32 rows and tokens per
+# CU (256) with row scales, four up to 64 tokens, five with per-block scales.
+@pytest.mark.parametrize("scales,rows,tokens,few", [
+    ("row", 4096, 16, True), ("row", 4096, 192, True), ("row", 4096, 193, False), ("row", 4096, 256, False),
+    ("row", 16384, 64, True), ("row", 16416, 64, False), ("row", 28672, 32, True), ("row", 28672, 33, False),
+    ("block", 4096, 320, True), ("block", 4096, 321, False), ("block", 28672, 32, True), ("block", 28672, 33, False),
+    ("unfolded", 4096, 2048, True)])
+def test_few_token_rule(scales, rows, tokens, few):
+    raw = synth.q8_matrix(3, rows, 64, synth.scale_base_for(64), scales == "row")
+    m = Q8Matrix.from_bytes(raw, rows, 64)
+    if scales == "block":
+        m.prepare_matrix_cores()
+    assert m.route(tokens).startswith("few") == few, m.route(tokens)
