@@ -310,10 +310,27 @@ static bool few_tiles(const GemvArgs& a) {
            (uint64_t)((a.w.tiles + 1) / 2) * ((a.tokens + 31) / 32) <= (uint64_t)per_cu * (uint32_t)iris_device_cus();
 }
 
+// The shape of a launch: tiles of 16 or 32 rows and tokens, and the waves
+// that share one's k steps.
+struct SkinnyLaunch {
+    uint32_t side, waves, row_tiles, tok_tiles;
+    // Groups of 8 row tiles, one per XCD, each with its token tiles in turn.
+    uint64_t blocks() const { return (uint64_t)(row_tiles + 7) / 8 * 8 * tok_tiles; }
+    uint64_t threads() const { return 64 * waves * blocks(); }
+};
+
+static SkinnyLaunch skinny_shape(const GemvArgs& a) {
+    const bool small = a.tokens <= 16;
+    const uint32_t row_tiles = small ? a.w.tiles : (a.w.tiles + 1) / 2, tok_tiles = (a.tokens + 31) / 32;
+    return {small ? 16u : 32u, (uint64_t)row_tiles * tok_tiles <= (uint32_t)iris_device_cus() ? 8u : 4u, row_tiles, tok_tiles};
+}
+
 bool iris_skinny_applies(const GemvArgs& a) {
     if (!a.planes || !a.token_limbs || a.tokens < 2 || a.w.cols % 64 || a.epilogue == EPI_HEAD_SELECT ||
         a.prologue == PRO_NORM_RES_NORM || a.tokens > 65535)
         return false;
+    // A launch holds fewer than 2^32 threads.
+    if (skinny_shape(a).threads() >> 32) return false;
     if (a.w.scale_mode == Q8_SCALE_ROW) return a.w.cols < (1u << 17) && few_tiles(a);
     // The planes' only path, whatever the tokens (two shared-shift terms).
     if (a.w.scale_mode == Q16_PLANES)
@@ -327,22 +344,10 @@ bool iris_skinny_applies(const GemvArgs& a) {
            a.w.cols <= 16384 && (few_tiles(a) || !a.w.fold_planes);
 }
 
-// The shape of a launch: tiles of 16 or 32 rows and tokens, and the waves
-// that share one's k steps.
-struct SkinnyLaunch {
-    uint32_t side, waves, row_tiles, tok_tiles;
-};
-
-static SkinnyLaunch skinny_shape(const GemvArgs& a) {
-    const bool small = a.tokens <= 16;
-    const uint32_t row_tiles = small ? a.w.tiles : (a.w.tiles + 1) / 2, tok_tiles = (a.tokens + 31) / 32;
-    return {small ? 16u : 32u, row_tiles * tok_tiles <= (uint32_t)iris_device_cus() ? 8u : 4u, row_tiles, tok_tiles};
-}
-
 int iris_skinny_launch(const GemvArgs& a, hipStream_t stream) {
     const SkinnyLaunch s = skinny_shape(a);
     const uint32_t row_tiles = s.row_tiles, tok_tiles = s.tok_tiles;
-    const dim3 grid((row_tiles + 7) / 8 * 8 * tok_tiles);
+    const dim3 grid((uint32_t)s.blocks());
     auto launch = [&](auto sh, auto w) {
         constexpr int SH = decltype(sh)::value;
         constexpr uint32_t W = decltype(w)::value;

@@ -639,7 +639,7 @@ static int i32_product(IrisSession* s, const I32GemvArgs& ig, const Q16Planes& p
     g.residual = ig.aux;
     g.residual_stride = ig.aux_stride;
     with_gemm_space(g, s, rows);
-    return iris_gemm_launch(g, s->stream);
+    return iris_gemm_applies(g) ? iris_gemm_launch(g, s->stream) : iris_i32_gemv_launch(ig, rows, s->stream);
 }
 
 static int gemma_ple(IrisSession* s, uint32_t rows) {

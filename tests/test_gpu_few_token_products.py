@@ -51,3 +51,11 @@ def test_few_token_rule(scales, rows, tokens, few):
     if scales == "block":
         m.prepare_matrix_cores()
     assert m.route(tokens).startswith("few") == few, m.route(tokens)
+
+
+def test_products_past_one_launch_stay_on_the_vector_path():
+    # 300000 unfolded rows and 60000 tokens (a 72 GB result) are 17.6 M tiles
+    # of 256 threads, past the 2^32 threads of a launch.
+    m = Q8Matrix.from_bytes(synth.q8_matrix(3, 300000, 64, synth.scale_base_for(64), False), 300000, 64)
+    assert m.route(50000) == "few 32x32, 4 waves"
+    assert m.route(60000) == "per token"
