@@ -89,10 +89,12 @@ int q8gpu_product_device_ws(const Q8GpuMatrix* matrix, const int32_t* d_activati
 
 /* Folds a per-block scale matrix's scales into weight digit planes so that
  * its multi-token products (q8gpu_product_device_ws, _noalloc and
- * q8gpu_product) run on the int8 matrix cores. Every matrix of finite
- * scales folds: 1 to Q8_FOLD_MAX_PLANES (6) planes, by how far a row's
- * scales spread (3 for the reference bundles' layout, 6 for a subnormal
- * block beside exponent 30). Allocates that many x rows x cols bytes more
+ * q8gpu_product) run on the int8 matrix cores: 1 to Q8_FOLD_MAX_PLANES (6)
+ * planes, by how far a row's scales spread (3 for the reference bundles'
+ * layout, 6 for a subnormal block beside exponent 30). Every matrix of finite
+ * scales folds but one with a row that holds a weight of -128 under scales of
+ * both signs of at least 65280 and a scale below 2^-13: that is left as
+ * uploaded. Allocates that many x rows x cols bytes more
  * device memory (reported by q8gpu_matrix_info's bytes; rows padded to a
  * multiple of 16), and synchronises `stream`. Does nothing, and returns 0, for a
  * row-scale matrix or one already prepared. Not to be called while other

@@ -21,33 +21,31 @@ namespace {
 // 5 * 2^28 < 2^31 for K <= 16384). The epilogue recombines the shifts in 128
 // bits, shifts by R and rounds once at 24 fraction bits.
 
+constexpr int32_t FOLD_NEGATED = 64;  // in a row's shift (0..29): its w' are kept negated
+
 // The signed byte digits of |v| < 2^47 (six bytes, d_l = byte l as int8,
-// v = sum_l 256^l d_l) and how many of them v needs.
+// v = sum_l 256^l d_l) and how many of them v needs: seven past the largest
+// value of six, 0x7f7f7f7f7f7f (the least is -0x808080808080).
 __device__ __forceinline__ uint64_t digits6(int64_t v) {
     return (uint64_t)(v + 0x808080808080LL) ^ 0x808080808080ULL;
 }
 __device__ __forceinline__ int digits6_needed(uint64_t d) {
-    return (d >> 40) ? 6 : (d >> 32) ? 5 : (d >> 24) ? 4 : (d >> 16) ? 3 : (d >> 8) ? 2 : 1;
+    return (d >> 48) ? 7 : (d >> 40) ? 6 : (d >> 32) ? 5 : (d >> 24) ? 4 : (d >> 16) ? 3 : (d >> 8) ? 2 : 1;
 }
 
-// Per row: R (the least exponent shift of its non-zero block scales; 0 for
-// an all-zero row) into shift[row], and the digits its largest |w'| needs
-// raised into *need (at most 6: sh_b - R <= 29, so |w'| < 2^47).
+// Per row, the digits its w' need (R the upload's shift[row]) raised into
+// *need. sh_b - R <= 29, so |w'| < 2^47, but a weight of -128 under a scale of
+// -65280 or more, beside a scale of the least exponent, passes six digits
+// (they reach further down than up): such a row is kept negated, marked in
+// shift[row], and only one that passes them either way needs the seventh.
 __global__ __launch_bounds__(256) void fold_rows_kernel(const uint8_t* qs, const uint16_t* sc16, uint32_t rows,
                                                         uint32_t nb, int32_t* shift, int* need) {
     const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= rows) return;
     const uint32_t tile = row / Q8_TILE_ROWS, r = row % Q8_TILE_ROWS;
     const uint16_t* sc = sc16 + (size_t)tile * nb * Q8_TILE_ROWS + r;
-    int least = 64;
-    for (uint32_t b = 0; b < nb; b++) {
-        const uint32_t bits = sc[(size_t)b * Q8_TILE_ROWS], e = (bits >> 10) & 0x1f, mant = bits & 0x3ff;
-        if (e == 0 && mant == 0) continue;
-        least = min(least, e ? (int)e - 1 : 0);
-    }
-    if (least == 64) least = 0;
-    shift[row] = least;
-    int digits = 1;
+    const int least = shift[row];
+    int digits = 1, negated = 1;
     const uint8_t* q = qs + (size_t)tile * nb * Q8_TILE_BLOCK_BYTES + r * 16;
     for (uint32_t b = 0; b < nb; b++) {
         const uint32_t bits = sc[(size_t)b * Q8_TILE_ROWS], e = (bits >> 10) & 0x1f, mant = bits & 0x3ff;
@@ -64,7 +62,14 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(const uint8_t* qs, const
                 qmin = min(qmin, v);
             }
         const int64_t f = (bits & 0x8000) ? -(m << d) : (m << d);
-        for (int64_t wv : {f * qmax, f * qmin}) digits = max(digits, digits6_needed(digits6(wv)));
+        for (int64_t wv : {f * qmax, f * qmin}) {
+            digits = max(digits, digits6_needed(digits6(wv)));
+            negated = max(negated, digits6_needed(digits6(-wv)));
+        }
+    }
+    if (digits > 6 && negated <= 6) {
+        shift[row] = least | FOLD_NEGATED;
+        digits = negated;
     }
     atomicMax(need, digits);
 }
@@ -81,8 +86,9 @@ __global__ __launch_bounds__(256) void fold_planes_kernel(const uint8_t* qs, con
     const uint32_t bits = sc16[((size_t)tile * nb + b) * Q8_TILE_ROWS + r], e = (bits >> 10) & 0x1f,
                    mant = bits & 0x3ff;
     const int64_t m = (int64_t)(e ? 1024 + mant : mant);
-    const int d = m ? (e ? (int)e - 1 : 0) - shift[row] : 0;
-    const int64_t f = (bits & 0x8000) ? -(m << d) : (m << d);
+    const int32_t sh = shift[row];
+    const int d = m ? (e ? (int)e - 1 : 0) - (sh & ~FOLD_NEGATED) : 0;
+    const int64_t f = !(bits & 0x8000) != !(sh & FOLD_NEGATED) ? -(m << d) : (m << d);
     const size_t off = ((size_t)tile * nb + b) * Q8_TILE_BLOCK_BYTES + r * 16;
     for (int h = 0; h < 2; h++) {
         const uint4 qv = *(const uint4*)(qs + off + h * 256);
@@ -196,11 +202,13 @@ __device__ __forceinline__ void fold_mainloop(const GemvArgs& a, int8_t* smem, u
 // The shared-shift sums recombine into sum_k w'_k x_k, shifted by the row's
 // R and rounded once at 24 fraction bits. In double the sum is exact below
 // 2^53 and the shift always, so the rounding to the nearest integer is the
-// only one; a wave with a larger sum redoes its block in 128 bits.
+// only one; a wave with a larger sum redoes its block in 128 bits. (A negated
+// row's sign comes back with the scale.)
 template <int NS>
 __device__ __forceinline__ void fold_values(const Q8View& w, uint32_t row, const v16i (&acc)[NS], int32_t (&v)[16]) {
-    const int32_t shift = row < w.rows ? w.fold_shift[row] : 0;
-    const double scale = __hiloint2double((1023 + shift - 24) << 20, 0);  // 2^(shift - 24)
+    const int32_t marked = row < w.rows ? w.fold_shift[row] : 0, shift = marked & ~FOLD_NEGATED;
+    const bool negated = marked & FOLD_NEGATED;
+    const double scale = __hiloint2double((negated ? 0x80000000u : 0) | (1023 + shift - 24) << 20, 0);  // +-2^(shift - 24)
     double most = 0;
 #pragma unroll
     for (int e = 0; e < 16; e++) {
@@ -217,6 +225,7 @@ __device__ __forceinline__ void fold_values(const Q8View& w, uint32_t row, const
         dn::i128 tot = 0;
 #pragma unroll
         for (int s = 0; s < NS; s++) tot += (dn::i128)((dn::u128)(dn::i128)acc[s][e] << (8 * s));
+        if (negated) tot = -tot;
         v[e] = dn::round_to_i32((dn::i128)((dn::u128)tot << shift), 24);
     }
 }

@@ -46,8 +46,8 @@ struct Q8Folded {
 
 // Weight digit planes of a folded matrix, at most: the widest spread of a
 // row's f16 scales (a subnormal block beside exponent 30, 29 binary orders)
-// makes |w'| <= 127 * 2047 * 2^29 < 2^47, six signed byte digits, so every
-// matrix with finite scales folds.
+// makes |w'| <= 128 * 2047 * 2^29 < 2^47, six signed byte digits, but for the
+// largest (fold_rows_kernel: kept negated, or the matrix is not folded).
 constexpr uint32_t Q8_FOLD_MAX_PLANES = 6;
 
 struct Q8GpuMatrix {

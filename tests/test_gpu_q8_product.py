@@ -340,6 +340,37 @@ def test_per_block_scales_on_the_matrix_cores(kind, planes, tokens, rows, cols):
     assert np.array_equal(dout.to_array(np.int32, (70, rows)), cpu.linear_q8(x2, raw))
 
 
+@pytest.mark.parametrize("signs", [(1,), (-1,), (1, -1)])
+def test_largest_folded_weights(signs):
+    # -128 under scales of 65280 and more, beside a subnormal scale: a
+    # negative one makes w' = 128 * (2040..2047) * 2^29, past the largest value
+    # of six signed byte digits (0x7f7f7f7f7f7f), a positive one fits, and a
+    # row with both cannot fold. One value of x per token, so that no result
+    # saturates, and full rows.
+    rng = np.random.default_rng(len(signs))
+    rows, cols, tokens = 72, 256, 70
+    raw = per_block_matrix(rng, rows, cols, "widest")
+    b = raw.reshape(rows, cols // 32, 34)
+    b[:, :, 2:][b[:, :, 2:] == 0x80] = 0x81  # -128 only where set below
+    for i, sign in enumerate(signs):
+        for r in (3, 16, 71):
+            b[r, 1 + i, 0], b[r, 1 + i, 1] = 0xF8 + r % 8, 0x7B | (0x80 if sign < 0 else 0)
+            b[r, 1 + i, 2 + r % 32] = 0x80
+            b[r, 0, :2] = 1, 0  # 2^-24
+    m = Q8Matrix.from_bytes(raw, rows, cols)
+    before = m.info()["bytes"]
+    m.prepare_matrix_cores()
+    folds = len(signs) == 1
+    assert m.info()["bytes"] - before == (6 * 80 * cols if folds else 0)
+    assert m.route(tokens) == ("folded 64x64, 6 planes" if folds else "per token")
+    x = np.zeros((tokens, cols), np.int32)
+    x[np.arange(64), 32 + np.arange(64)] = rng.integers(50, 250, 64)
+    x[64:] = rng.integers(-2000, 2000, (tokens - 64, cols))
+    want = cpu.linear_q8(x, raw)
+    assert 0 < np.abs(want[3 % 32, 3].astype(np.int64)) < 2 ** 31 - 1
+    assert np.array_equal(product_ws(m, x), want)
+
+
 def test_per_block_gemm_at_the_benchmark_shape_sampled():
     # The gate|up shape of the 2048-row pass with per-block scales (the
     # reference bundles' layout: base + next % 64 significands, generate.py:59):
