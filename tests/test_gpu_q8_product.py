@@ -212,13 +212,11 @@ def grouped_activations(rng, tokens, cols):
                                               (603, 136, 8192)])
 def test_mfma_product_digit_paths(tokens, rows, cols):
     # Every digit count's code path (one to three planes side by side, four
-    # and five in two token halves), one-step, short and long k loops,
+    # and five in passes of their own), one-step, short and long k loops, and
     # launches whose block count does and does not split evenly over the
-    # XCDs, and both workgroup shapes (256-row blocks when the launch fills
-    # every CU: the fourth and fifth cases). The 128-row shapes split an
-    # even number of 64-wide k steps between two wave groups (the last three
-    # cases; rows of 8192 or more take the deeper rings, three stages at
-    # three planes) and walk an odd number in one (the first three).
+    # XCDs. (300, 22100, 128) and (200, 32768, 64) take the tiled products,
+    # the others the few-token one; test_gpu_gemm_tiles.py has every tiled
+    # shape by name.
     rng = np.random.default_rng(tokens + rows + cols)
     raw = synth.q8_matrix(synth.tensor_seed(11, rows), rows, cols, synth.scale_base_for(cols), True)
     m = Q8Matrix.from_bytes(raw, rows, cols)
@@ -236,9 +234,8 @@ def test_mfma_product_digit_paths(tokens, rows, cols):
 def test_mfma_product_wide_row_scales():
     # Row-scale matrices whose Q.24 scales run from zero and subnormals up to
     # f16 exponent 30 (about 2^40), both signs, against full-range
-    # activations with every magnitude from 8 to 32 bits: the MFMA epilogue's
-    # 64-bit rounding path, its bit-length test near 2^63 and its 128-bit
-    # redo all run; every output is compared.
+    # activations with every magnitude from 8 to 32 bits, through the
+    # few-token product; every output is compared.
     rng = np.random.default_rng(31)
     rows, cols, tokens = 512, 1024, 96
     nb = cols // 32
@@ -302,7 +299,9 @@ def per_block_matrix(rng, rows, cols, kind):
 @pytest.mark.parametrize("tokens,rows,cols", [(603, 200, 128), (129, 136, 4160)])
 def test_per_block_scales_on_the_matrix_cores(kind, planes, tokens, rows, cols):
     # Per-block scale matrices folded into weight digit planes for the int8
-    # matrix cores, one to six planes (every spread an f16 scale row can
+    # matrix cores (up to three planes these shapes stay on the few-token
+    # product all the same; test_gpu_gemm_tiles.py has larger ones), one to
+    # six planes (every spread an f16 scale row can
     # have folds): every digit count of the activations (token groups of
     # 1..5 digits), partial row and token tiles, every output against the
     # oracle's dot_row. (None: the count depends on the draw.)
@@ -317,7 +316,8 @@ def test_per_block_scales_on_the_matrix_cores(kind, planes, tokens, rows, cols):
     assert before == padded * (cols + cols // 32 * 2 + 4)
     x = grouped_activations(rng, tokens, cols)
     want = cpu.linear_q8(x, raw)
-    # Unprepared: the vector path, and the product allocates nothing.
+    # Unprepared: up to three weight digits the few-token product, else the
+    # vector path; the product allocates nothing.
     assert np.array_equal(product_ws(m, x), want)
     assert m.info()["bytes"] == before
     m.prepare_matrix_cores()
