@@ -247,6 +247,14 @@ extern "C" {
         weight_out: *mut i32,
         score_out: *mut i32,
     ) -> c_int;
+    pub fn iris_score_numerics(
+        dot: *const i64,
+        scaled: c_int,
+        scale_q32: u32,
+        n: u32,
+        score_out: *mut i32,
+        quick_out: *mut i32,
+    ) -> c_int;
     pub fn iris_silu_device(x: *const i32, n: u32, out: *mut i32) -> c_int;
     pub fn iris_silu_table_device(x: *const i32, n: u32, out: *mut i32) -> c_int;
     pub fn iris_sha256_bytes(data: *const u8, len: u64, out: *mut u8) -> c_int;

@@ -370,14 +370,23 @@ int iris_attention_numerics(const uint32_t* diff, const uint64_t* e, const uint6
                             uint32_t scale_q32, uint32_t n, uint64_t* exp_out, int32_t* weight_out,
                             int32_t* score_out);
 
+/* Numerics check: the attention score of each dot product dot[i] as the
+ * matrix-core attention forms it from its sum in double, scaled by scale_q32
+ * (scaled != 0) or requantized; quick_out[i] is 0 where the exact routine
+ * decided (device pointers; synchronous). No counterpart in the reference: it
+ * compares the score with scaled_score (crates/det-num/src/mistral.rs:130-145)
+ * and requantize (crates/det-num/src/ops.rs:448-451). */
+int iris_score_numerics(const int64_t* dot, int scaled, uint32_t scale_q32, uint32_t n, int32_t* score_out,
+                        int32_t* quick_out);
+
 /* Numerics check: silu (crates/det-num/src/mistral.rs:59-77, the SwiGLU
  * gate) of n Q16.16 values on the device, as the product epilogues compute
  * it (device pointers; synchronous). No counterpart in the reference. */
 int iris_silu_device(const int32_t* x, uint32_t n, int32_t* out);
 
-/* Numerics check: the same silu through the device's silu table, as the
- * matrix-core SwiGLU epilogues look it up (device pointers; synchronous; the
- * table is made on the first call on a device). No counterpart in the
+/* Numerics check: the same silu as the matrix-core SwiGLU epilogues form it,
+ * in double and near a rounding tie from the device's silu table (device
+ * pointers; synchronous; the table is made on the first call on a device). No counterpart in the
  * reference. */
 int iris_silu_table_device(const int32_t* x, uint32_t n, int32_t* out);
 

@@ -219,6 +219,14 @@ __device__ __forceinline__ void load_key_tile(const int8_t* kb, size_t kl, v4i (
 // The scores of one 16-key tile against the wave's 16 query rows, from LQK
 // digit planes of each: lane l holds query l % 16 and keys 4 * (l / 16) + i
 // of the tile.
+// A score from its sum in double (scale = scale_q32 * 2^-48). False: the
+// exact routine decides (near a rounding tie, or the sum may not be exact).
+__device__ __forceinline__ bool quick_score(bool scaled, double s, double scale, int32_t& sc) {
+    if (scaled) return dn::scaled_score_fast(s, scale, sc);
+    sc = dn::requantize((int64_t)s);
+    return fabs(s) < 0x1p53;
+}
+
 template <uint32_t HD, int LQK>
 __device__ __forceinline__ void tile_scores(const AttnArgs& a, const v4i (&kf)[LQK][HD / 64],
                                             const v4i (&qf)[LQK][HD / 64], int32_t (&sc)[4]) {
@@ -257,12 +265,7 @@ __device__ __forceinline__ void tile_scores(const AttnArgs& a, const v4i (&kf)[L
                 const int32_t pair = j + 1 < NS ? acc[j][i] + (acc[j + 1][i] << 8) : acc[j][i];
                 s = fma(s, 65536.0, (double)pair);
             }
-            if (a.scaled) {
-                slow |= !dn::scaled_score_fast(s, scale, sc[i]);
-            } else {
-                sc[i] = dn::requantize((int64_t)s);
-                slow |= fabs(s) >= 0x1p53;  // no longer exact
-            }
+            slow |= !quick_score(a.scaled, s, scale, sc[i]);
         }
         if (!__any(slow)) return;
     }
@@ -719,7 +722,29 @@ __global__ void attention_numerics_kernel(const uint32_t* diff, const uint64_t* 
     score_out[i] = dn::scaled_score_from_sum(dot[i], scale_q32);
 }
 
+__global__ void score_numerics_kernel(const int64_t* dot, int scaled, uint32_t scale_q32, uint32_t n, int32_t* score_out,
+                                      int32_t* quick_out) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    int32_t sc;
+    const bool quick = quick_score(scaled, (double)dot[i], (double)scale_q32 * 0x1p-48, sc);
+    if (!quick) sc = scaled ? dn::scaled_score_from_sum(dot[i], scale_q32) : dn::requantize(dot[i]);
+    score_out[i] = sc;
+    quick_out[i] = quick;
+}
+
 }  // namespace
+
+int iris_score_numerics(const int64_t* d_dot, int scaled, uint32_t scale_q32, uint32_t n, int32_t* d_score,
+                        int32_t* d_quick) {
+    if (n == 0) return 0;
+    if (!d_dot || !d_score || !d_quick) return IRIS_E_INVALID;
+    hipLaunchKernelGGL(score_numerics_kernel, dim3((n + 255) / 256), dim3(256), 0, nullptr, d_dot, scaled, scale_q32, n,
+                       d_score, d_quick);
+    hipError_t st = hipGetLastError();
+    if (st == hipSuccess) st = hipDeviceSynchronize();
+    return (int)st;
+}
 
 int iris_attention_numerics(const uint32_t* d_diff, const uint64_t* d_e, const uint64_t* d_sum, const int64_t* d_dot,
                             uint32_t scale_q32, uint32_t n, uint64_t* d_exp, int32_t* d_weight, int32_t* d_score) {

@@ -75,6 +75,7 @@ def _declare(L):
         "iris_time_product": (C.c_int, [vp, u32, vp, u32, vp, u32, C.POINTER(C.c_double)]),
         "iris_time_bcast_product": (C.c_int, [vp, u32, vp, vp, u32, C.POINTER(C.c_double)]),
         "iris_attention_numerics": (C.c_int, [vp, vp, vp, vp, u32, u32, vp, vp, vp]),
+        "iris_score_numerics": (C.c_int, [vp, C.c_int, u32, u32, vp, vp]),
         "iris_silu_device": (C.c_int, [vp, u32, vp]),
         "iris_silu_table_device": (C.c_int, [vp, u32, vp]),
         "iris_time_product_ws": (C.c_int, [vp, vp, u32, vp, vp, u64, u32, C.POINTER(C.c_double)]),

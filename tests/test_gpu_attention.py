@@ -69,6 +69,43 @@ def test_attention_numerics_against_oracle():
     assert np.array_equal(got_s[idx], want_s)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128, 0])
+def test_scores_in_double_against_oracle(head_dim):
+    # Sums around every kind of rounding tie, scaled (head sizes 64 and 128)
+    # and unscaled (0): 40 units to either side of sums whose score is a half
+    # integer (the tie window of a scaled score is 16 units or more, so both
+    # its edges), near zero, through the range, at both ends of the i32 range
+    # and past them up to the largest sums of three-digit operands (2^53 and a
+    # little over), and random ones. The exact routine decides inside the
+    # window and for unscaled sums past 2^53, the double elsewhere.
+    O = cpu.lib()
+    scale = O.dn_attention_scale_q32(head_dim) if head_dim else 0
+    unit = 2 ** 48 / scale if head_dim else 2 ** 16  # sums a score apart
+    rng = np.random.default_rng(head_dim)
+    n = np.r_[np.arange(-40, 40), rng.integers(-2 ** 31, 2 ** 31, 200), 2 ** 31 + np.arange(-6, 6),
+              -2 ** 31 + np.arange(-6, 6), [2 ** 33, -2 ** 33]].astype(np.int64)
+    ties = np.array([int((2 * int(v) + 1) * unit / 2) for v in n], np.int64)
+    ends = np.array([2 ** 53, -2 ** 53, 2 ** 53 + 2 ** 46, -2 ** 53 - 2 ** 46], np.int64)
+    dots = np.r_[(np.r_[ties, ends][:, None] + np.arange(-40, 41)).ravel(), rng.integers(-2 ** 53, 2 ** 53, 4000),
+                 rng.integers(-2 ** 40, 2 ** 40, 4000)]
+    dots = dots[np.abs(dots) < 2 ** 54]
+    d, score, quick = native.DeviceBuffer.from_array(dots), native.DeviceBuffer(4 * dots.size), \
+        native.DeviceBuffer(4 * dots.size)
+    native.check(native.lib().iris_score_numerics(d.ptr, int(head_dim != 0), scale, dots.size, score.ptr, quick.ptr),
+                 "scores")
+    got, by_double = score.to_array(np.int32, (dots.size,)), quick.to_array(np.int32, (dots.size,))
+    if head_dim:
+        q = np.stack([dots >> 24, dots & 0xFFFFFF], 1).astype(np.int32)  # q . (2^24, 1) is the sum
+        k = np.array([1 << 24, 1], np.int32)
+        want = np.array([O.dn_scaled_score(row, k, 2, scale) for row in q], np.int32)
+    else:
+        want = np.array([O.dn_requantize(int(v)) for v in dots], np.int32)
+        assert np.array_equal(by_double != 0, np.abs(dots) < 2 ** 53)
+    assert np.array_equal(got, want)
+    assert 0 < np.count_nonzero(by_double) < dots.size
+    assert want.max() == 2 ** 31 - 1 and want.min() == -2 ** 31
+
+
 def _check_pass(m, rows, max_positions=None):
     ids = synth.token_ids(11, rows, m.vocab)
     dm = DeviceModel(m)
@@ -164,9 +201,9 @@ def test_long_context_decode_matches_oracle(family):
 @pytest.mark.timeout(600)
 def test_silu_every_input():
     # All 2^32 Q16.16 inputs, in chunks of 2^25: the device silu (the SwiGLU
-    # gate of the product epilogues) and the table lookup of the matrix-core
-    # epilogues (the table inside |x| < 1453635, x or 0 outside) against the
-    # oracle's silu (mistral.rs:59-77).
+    # gate of the one-row products) and that of the matrix-core epilogues
+    # (double arithmetic, the table near a rounding tie) against the oracle's
+    # silu (mistral.rs:59-77).
     chunk = 1 << 25
     dx = native.DeviceBuffer(4 * chunk)
     dout = native.DeviceBuffer(4 * chunk)
