@@ -67,11 +67,6 @@ __global__ __launch_bounds__(256) void token_prep_kernel(const GemvArgs a) {
     a.token_limbs[t] = dn::rms_scale_from_sum(s, a.w.cols, a.norm_eps);
 }
 
-__global__ __launch_bounds__(256) void fill_ints_kernel(int32_t* p, uint32_t n, int32_t v) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 // The digit planes of one 32-token tile over PLANE_KB k blocks (one k
 // chunk) per workgroup, after the optional rms_norm (mul_sat(mul_sat(v,
 // scale), w)), in the operand layout above, and the digits the chunk's
@@ -150,7 +145,9 @@ int iris_gemm_launch(const GemvArgs& a, hipStream_t stream) {
     if (!iris_gemm_applies(a) || a.x_stride % 4 || ((uintptr_t)a.x & 15) || ((uintptr_t)a.planes & 255))
         return IRIS_E_INVALID;
     if (a.prologue == PRO_RMSNORM && ((uintptr_t)a.norm_w & 15)) return IRIS_E_INVALID;
-    if (a.planes_ready && a.prologue != PRO_NONE) return IRIS_E_INVALID;
+    // (Ready planes are the down product's: what sets the gated rows' counts
+    // is the launch that makes the planes.)
+    if (a.planes_ready && (a.prologue != PRO_NONE || a.out_gemm_planes)) return IRIS_E_INVALID;
     const bool gated = a.epilogue == EPI_SWIGLU || a.epilogue == EPI_GEGLU;
     if (a.out_gemm_planes && (!gated || !a.out_gemm_limbs || (a.w.rows / 2) % 32 || ((uintptr_t)a.out_gemm_planes & 255) ||
                               a.out_gemm_planes == a.planes || a.out_gemm_limbs == a.token_limbs))
@@ -165,9 +162,6 @@ int iris_gemm_launch(const GemvArgs& a, hipStream_t stream) {
         const dim3 grid(TT, (KB + PLANE_KB - 1) / PLANE_KB);
         const bool few = grid.x * grid.y <= 2 * (uint32_t)iris_device_cus();
         hipLaunchKernelGGL(digit_planes_kernel, grid, dim3(few ? DP_THREADS : 256), 0, stream, a, ones);
-    } else if (ones) {
-        hipLaunchKernelGGL(fill_ints_kernel, dim3((ones + 255) / 256), dim3(256), 0, stream, a.out_gemm_limbs + a.tokens,
-                           ones, 1);
     }
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return (int)st;

@@ -241,10 +241,10 @@ __device__ __forceinline__ void fold_pass(const GemvArgs& a, int8_t* smem, uint3
     fold_mainloop<G, WP, LG>(a, smem, rt0, tt0, acc);
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t rt = rt0 + (wave % G::WR) * G::RI;
-    finish_blocks<G::RI, 1>(a, (int32_t*)smem + wave * G::RI * PARK_BLOCK, rt, tt0 + wave / G::WR,
-                            [&](int i, int, int32_t (&v)[16]) __attribute__((always_inline)) {
-                                fold_values<G::NS>(a.w, (rt + i) * 32 + lane % 32, acc[i], v);
-                            });
+    finish_blocks<G::RI>(a, (int32_t*)smem + wave * G::RI * PARK_BLOCK, rt, tt0 + wave / G::WR,
+                         [&](int i, int32_t (&v)[16]) __attribute__((always_inline)) {
+                             fold_values<G::NS>(a.w, (rt + i) * 32 + lane % 32, acc[i], v);
+                         });
 }
 
 // 32 * RT folded weight rows x 32 * TG tokens per workgroup.

@@ -215,10 +215,10 @@ __device__ __forceinline__ void gemm_pass(const GemvArgs& a, int8_t* smem, uint3
         first = second ? NI : 0;
     }
     const uint32_t rt = rt0 + (hw % WR) * RI + first;
-    finish_blocks<NI, 1>(a, (int32_t*)smem + wave * NI * PARK_BLOCK, rt, tt0 + hw / WR,
-                         [&](int i, int, int32_t (&v)[16]) __attribute__((always_inline)) {
-                             row_values<LG>(a.w, (rt + i) * 32 + lane % 32, acc[i], v);
-                         });
+    finish_blocks<NI>(a, (int32_t*)smem + wave * NI * PARK_BLOCK, rt, tt0 + hw / WR,
+                      [&](int i, int32_t (&v)[16]) __attribute__((always_inline)) {
+                          row_values<LG>(a.w, (rt + i) * 32 + lane % 32, acc[i], v);
+                      });
 }
 
 // 32W weight rows x 32 * TG tokens per workgroup. Up to three digit planes (the

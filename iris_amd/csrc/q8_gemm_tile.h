@@ -194,46 +194,43 @@ __device__ __forceinline__ void finish_parked(const GemvArgs& a, int32_t* block,
     for (uint32_t r = 0; r < n; r++) store_output(a, row0 + r, token, p[r], p[r ^ 1]);
 }
 
-// A wave's NI x NJ finished blocks (32-row tiles rt.., 32-token tiles tt..),
-// block (i, j) from values(i, j, v): from registers for a plain or residual
-// store, else through `park` (NI * NJ * PARK_BLOCK ints of the wave's own).
-template <int NI, int NJ, class Values>
+// A wave's NI finished blocks (32-row tiles rt.., 32-token tile tt), block i
+// from values(i, v): from registers for a plain or residual store, else
+// through `park` (NI * PARK_BLOCK ints of the wave's own).
+template <int NI, class Values>
 __device__ __forceinline__ void finish_blocks(const GemvArgs& a, int32_t* park, uint32_t rt, uint32_t tt, Values&& values) {
     const uint32_t lane = threadIdx.x & 63;
     const bool residual = a.epilogue == EPI_RESIDUAL, direct = residual || a.epilogue == EPI_STORE;
 #pragma unroll
-    for (int i = 0; i < NI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            int32_t v[16];
-            values(i, j, v);
-            if (direct) {
-                const uint32_t row = (rt + i) * 32 + lane % 32, tok0 = (tt + j) * 32 + 4 * (lane / 32);
-                if (row < a.w.rows) {
-                    if (residual) {
-#pragma unroll
-                        for (int e = 0; e < 16; e++) {
-                            const uint32_t token = min(tok0 + 8 * (e / 4) + e % 4, a.tokens - 1);
-                            v[e] = dn::add_sat(v[e], a.residual[(size_t)token * a.residual_stride + row]);
-                        }
-                    }
+    for (int i = 0; i < NI; i++) {
+        int32_t v[16];
+        values(i, v);
+        if (direct) {
+            const uint32_t row = (rt + i) * 32 + lane % 32, tok0 = tt * 32 + 4 * (lane / 32);
+            if (row < a.w.rows) {
+                if (residual) {
 #pragma unroll
                     for (int e = 0; e < 16; e++) {
-                        const uint32_t token = tok0 + 8 * (e / 4) + e % 4;
-                        if (token < a.tokens) a.out[(size_t)token * a.out_stride + row] = v[e];
+                        const uint32_t token = min(tok0 + 8 * (e / 4) + e % 4, a.tokens - 1);
+                        v[e] = dn::add_sat(v[e], a.residual[(size_t)token * a.residual_stride + row]);
                     }
                 }
-            } else {
 #pragma unroll
-                for (int e = 0; e < 16; e++)
-                    park[(i * NJ + j) * PARK_BLOCK + (2 * e + lane / 32) * PARK_LINE + lane % 32] = v[e];
+                for (int e = 0; e < 16; e++) {
+                    const uint32_t token = tok0 + 8 * (e / 4) + e % 4;
+                    if (token < a.tokens) a.out[(size_t)token * a.out_stride + row] = v[e];
+                }
             }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; e++) park[i * PARK_BLOCK + (2 * e + lane / 32) * PARK_LINE + lane % 32] = v[e];
         }
+    }
     if (direct) return;
     // The wave's own LDS: its accesses stay in order, the compiler keeps them so.
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll 1
-    for (uint32_t b = 0; b < NI * NJ; b++) finish_parked(a, park + b * PARK_BLOCK, rt + b / NJ, tt + b % NJ);
+    for (uint32_t b = 0; b < NI; b++) finish_parked(a, park + b * PARK_BLOCK, rt + b, tt);
 }
 
 // The nearest integer to an exact double, ties to even, saturated.
