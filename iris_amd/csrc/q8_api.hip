@@ -285,8 +285,9 @@ uint64_t q8gpu_workspace_bytes(const Q8GpuMatrix* m, uint32_t tokens) {
 }  // extern "C"
 
 // The product with optional work space. A per-block scale matrix takes the
-// matrix cores only once q8gpu_prepare_matrix_cores has folded it; nothing
-// here allocates, synchronises or changes the matrix.
+// matrix cores as uploaded where three weight digits suffice, else once
+// q8gpu_prepare_matrix_cores has folded it; nothing here allocates,
+// synchronises or changes the matrix.
 static int product_with_space(const Q8GpuMatrix* m, const int32_t* d_act, uint32_t tokens, int32_t* d_out,
                               void* d_workspace, uint64_t workspace_bytes, void* stream) {
     if (!m || (tokens && (!d_act || !d_out))) return IRIS_E_INVALID;
@@ -320,9 +321,9 @@ int q8gpu_prepare_matrix_cores(Q8GpuMatrix* m, void* stream) {
 }
 
 // q8gpu_product_device_ws with the device's scratch array as the work space:
-// no allocation of any kind. The digit counts are reset per token and every
-// plane of the used region is written by the call itself before it is read,
-// so nothing carried over from an earlier call is used.
+// no allocation of any kind. Every digit count, one per (k chunk, 32-token
+// tile), and every plane of the used region is written by the call itself
+// before it is read, so nothing carried over from an earlier call is used.
 int q8gpu_product_device_noalloc(const Q8GpuMatrix* m, const int32_t* d_act, uint32_t tokens, int32_t* d_out,
                                  void* stream) {
     if (!m || (tokens && (!d_act || !d_out))) return IRIS_E_INVALID;

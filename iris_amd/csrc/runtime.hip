@@ -612,12 +612,6 @@ static int mistral_pass(IrisSession* s, uint32_t rows, const CkptSink* sink) {
     return 0;
 }
 
-// One gemma-dense pass (crates/inference/kernels/src/prefill_range.rs:307-958
-// per layer, the PLE prepare of view_kernels.rs:59-99 first): eleven launches
-// per layer, eight for one row.
-//
-// The PLE inputs of every layer (view_kernels.rs:59-99) from the embedded
-// rows in s->x and their ids, into s->ple_rows [rows][layers * ple_width].
 // A Q16.16 product of a pass: on the matrix cores where its planes were
 // built and the rows are enough, else one row at a time. us of a prompt pass
 // of three Gemma-2B-shape layers (seven such products), row by row / planes:
@@ -642,6 +636,8 @@ static int i32_product(IrisSession* s, const I32GemvArgs& ig, const Q16Planes& p
     return iris_gemm_applies(g) ? iris_gemm_launch(g, s->stream) : iris_i32_gemv_launch(ig, rows, s->stream);
 }
 
+// The PLE inputs of every layer (view_kernels.rs:59-99) from the embedded
+// rows in s->x and their ids, into s->ple_rows [rows][layers * ple_width].
 static int gemma_ple(IrisSession* s, uint32_t rows) {
     IrisModel* m = s->model;
     const IrisModelDesc& d = m->d;
@@ -894,6 +890,9 @@ static bool gemma_carries(const IrisSession* s, uint32_t rows, const CkptSink* s
            H <= 4096 && H <= I32_GEMV_MAX_STAGED;
 }
 
+// One gemma-dense pass (crates/inference/kernels/src/prefill_range.rs:307-958
+// per layer, the PLE prepare of view_kernels.rs:59-99 first): eleven launches
+// per layer, eight for one row (attention counted once, preparations not).
 static int gemma_pass(IrisSession* s, uint32_t rows, const CkptSink* sink) {
     const bool carry = gemma_carries(s, rows, sink);
     s->carry = IrisSession::GemmaCarry{};
